@@ -194,15 +194,18 @@ Operand hc_operand(const void* h, const int64_t strides[3], int neg, int dtype) 
   return make_operand(h, strides, neg, dtype, 0);
 }
 
-int64_t resident_blocks(const void* kernel, int block) {
+int64_t compute_units() {
   int device = 0;
-  int per_cu = 0;
   int cus = 0;
   if (hipGetDevice(&device) != hipSuccess) return 1;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 1;
+  return cus > 0 ? cus : 1;
+}
+
+int64_t resident_blocks(const void* kernel, int block) {
+  int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) per_cu = 1;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 1;
-  const int64_t n = static_cast<int64_t>(per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1);
-  return n > 0 ? n : 1;
+  return (per_cu > 0 ? per_cu : 1) * compute_units();
 }
 
 }  // namespace fh

@@ -8,6 +8,8 @@ namespace fh {
 // Workgroups of `block` threads of `kernel` the current device holds at once
 // (occupancy x compute units); at least 1.
 int64_t resident_blocks(const void* kernel, int block);
+// Compute units of the current device; at least 1.
+int64_t compute_units();
 
 // One wavefront per matrix, reference evaluation order (checking aid).
 hipError_t launch_generic(const ExpmArgs& args, int dtype, int P, bool pair, hipStream_t stream);

@@ -6,28 +6,38 @@
 // fuses this; its matrix_exp (ops/matrix_exp/__init__.py:80-97) returns
 // exp(H) to the caller, who multiplies.  Here exp(H_b) never leaves the chip:
 //
-// * A wavefront takes a set of kTokens tokens spread over the batch: set k of
-//   S = ceil(B / kTokens) holds tokens k, k + S, k + 2S, ..., so wavefronts
-//   running at the same time stream neighbouring tokens and the rows in flight
-//   form one contiguous region of HBM (consecutive tokens per wavefront put
-//   every concurrent access 8 tokens apart, a power-of-two stride that costs
-//   about 15% of the bandwidth).  Lane l computes exp(H) of the set's token
-//   l % kTokens with the per-lane P == 4 code (p4_lane.h, the same arithmetic
-//   as the matrix-exponential kernel, so E is bit-identical to it) and parks
-//   it in the wavefront's LDS.
-// * The wavefront then streams each token's rows: every lane loads 16 bytes
-//   of each of the n rows per chunk (the whole wavefront covers 1 KB of each
-//   row per chunk, coalesced), multiplies by E read back from LDS (one
+// * A workgroup of four wavefronts takes a set of T tokens spread over the
+//   batch: set k of S = ceil(B / T) holds tokens k, k + S, k + 2S, ..., so
+//   workgroups running at the same time stream neighbouring tokens and the rows
+//   in flight form one contiguous region of HBM (consecutive tokens per
+//   workgroup put every concurrent access T tokens apart, a power-of-two stride
+//   that costs about 15% of the bandwidth).  T follows the batch (launch_sets):
+//   8 or 16 when there are tokens enough to fill the chip that way, down to one
+//   token a workgroup.  One wavefront to 8 tokens, however few there were, left
+//   most of the chip idle below 16384 tokens: 64 x 4 x 4096 BF16 forward 61 ->
+//   6.3 us, 2048 x 4 x 4096 forward 80 -> 27 us and backward 132 -> 47 us,
+//   2048 x 8 x 4096 forward 162 -> 50 us and backward 289 -> 79 us.
+// * The wavefronts split each token's columns between them, 64 lanes' chunks in
+//   turn (column_parts), so that one token already keeps four wavefronts
+//   streaming.  The split depends on C alone, so a token's results do not
+//   depend on the batch.
+// * Lane l of every wavefront computes exp(H) of the set's token l with the
+//   per-lane P == 4 code (p4_lane.h, the same arithmetic as the
+//   matrix-exponential kernel, so E is bit-identical to it) and parks it in the
+//   wavefront's own LDS.
+// * A wavefront then streams its columns of each token: every lane loads 16
+//   bytes of each of the n rows per chunk (the whole wavefront covers 1 KB of
+//   each row per chunk, coalesced), multiplies by E read back from LDS (one
 //   broadcast read per token) and stores 16 bytes of each output row.  Rows
 //   are read and written once, with the nontemporal cache hint.  Rows
 //   are addressed through a buffer resource rebased per token in SGPRs, so no
 //   VALU address arithmetic is needed and offsets never exceed one token.
 // * The backward accumulates dE_b = dY_b X_b^T per lane over its columns (in
 //   column order), reduces the 16 partial sums across the wavefront with a
-//   fixed exchange tree (the result does not depend on anything but the
-//   data), parks dE_b in LDS, and after its tokens each lane runs the P == 4
-//   Frechet polynomial on (H^T, dE) of one token -- the same arithmetic as the
-//   Frechet kernel.
+//   fixed exchange tree, adds the wavefronts' parts in order through LDS (the
+//   result does not depend on anything but the data), and after the set's
+//   tokens each lane of one wavefront runs the P == 4 Frechet polynomial on
+//   (H^T, dE) of one token -- the same arithmetic as the Frechet kernel.
 //
 // Both directions are bound by HBM traffic (16 FMAs per 2n elements moved
 // forward, 32 per 3n backward); the exponential and Frechet work per token is
@@ -39,8 +49,8 @@ namespace {
 
 using namespace p4;
 
-constexpr int kWaves = 4;   // wavefronts per workgroup
-constexpr int kTokens = 8;  // tokens per wavefront
+constexpr int kWaves = 4;    // wavefronts per workgroup
+constexpr int kTokens = 16;  // tokens per workgroup, at most
 
 struct HcArgs {
   Operand h;        // [B, n, n]
@@ -53,6 +63,9 @@ struct HcArgs {
   float* aux;       // optional FP32 [B, n, n]: exp(H) (forward) or dE (backward)
   int64_t batch;
   int64_t cols;
+  int64_t sets;     // workgroups
+  int tokens;       // per workgroup
+  int parts;        // wavefronts that share a token's columns (column_parts)
   int n;
 };
 
@@ -113,16 +126,35 @@ __device__ __forceinline__ void store16(U32x4 w, __amdgpu_buffer_rsrc_t rs, int3
   __builtin_amdgcn_raw_buffer_store_b128(w, rs, voff, 0, kStreamPolicy);
 }
 
-// Token set `k` of `sets` = ceil(batch / kTokens): tokens k + i * sets, i < count.
-struct TokenSet {
-  int64_t first, stride;
-  int count;
-  __device__ __forceinline__ int64_t token(int i) const { return first + i * stride; }
+// Wavefronts of a workgroup that share one token's columns, for passes of
+// `width` columns: four, or fewer when C has fewer passes, in which case the
+// others take other tokens.  By C alone (see above).
+int column_parts(int64_t cols, int64_t width) {
+  const int64_t passes = cols / width;
+  return passes >= 4 ? 4 : passes >= 2 ? 2 : 1;
+}
+
+// A workgroup's set of tokens, slots 0 .. slots - 1, and a wavefront's share of
+// it.  `parts` wavefronts share a token's columns, in passes of chunks part,
+// part + parts, ...; abreast = kWaves / parts tokens run side by side in slots
+// first, first + abreast, ....  Slots side by side hold neighbouring tokens,
+// slots after one another tokens sets * abreast apart; the set's last slots may
+// lie past the batch.
+struct Share {
+  int64_t base, stride;  // token of slot i: base + i % abreast + i / abreast * stride
+  int64_t batch;
+  int slots, abreast, shift, parts, first, part;  // abreast = 1 << shift
+  __device__ __forceinline__ int64_t token(int i) const { return base + (i & (abreast - 1)) + (i >> shift) * stride; }
+  __device__ __forceinline__ bool holds(int i) const { return i < slots && token(i) < batch; }
+  __device__ __forceinline__ int column(int chunk, int width) const { return (chunk * parts + part) * width; }
 };
 
-__device__ __forceinline__ TokenSet token_set(int64_t k, int64_t sets, int64_t batch) {
-  const int64_t left = (batch - k + sets - 1) / sets;
-  return TokenSet{k, sets, static_cast<int>(left < kTokens ? left : kTokens)};
+template <typename Args>
+__device__ __forceinline__ Share share_of(const Args& a, int wave) {
+  static_assert(kWaves == 4, "parts is 1, 2 or 4");
+  const int shift = a.parts == 4 ? 0 : a.parts == 2 ? 1 : 2;
+  return Share{static_cast<int64_t>(blockIdx.x) << shift, a.sets << shift, a.batch, a.tokens, 1 << shift, shift,
+               a.parts, wave >> (2 - shift), wave & (a.parts - 1)};
 }
 
 // exp(H) of token `b` for this lane (valid lanes), NaN for a non-finite H
@@ -145,21 +177,20 @@ __device__ __forceinline__ M4 exp_of_token(const Operand& h, int64_t b, bool val
   return e;
 }
 
-// The wavefront's token set: lane l holds exp(H) of token l % kTokens of the
-// set and lanes below kTokens park it in `etile` (16 floats per token); `aux`
-// (optional) receives it in FP32.
+// exp(H) of the set's tokens into the wavefront's `etile` (16 floats per
+// token): lane l computes token l (lanes past the set a zero matrix).  `aux`
+// (optional) receives it in FP32 from the first wavefront.
 template <typename T, int N>
-__device__ __forceinline__ void exp_tokens(const HcArgs& a, const TokenSet& ts, int lane, float* etile) {
-  const int slot = lane & (kTokens - 1);
-  const int64_t b = ts.token(slot);
-  const bool valid = slot < ts.count;
+__device__ __forceinline__ void exp_tokens(const HcArgs& a, const Share& sh, int lane, int wave, float* etile) {
+  const bool valid = sh.holds(lane);
+  const int64_t b = sh.token(lane);
   const M4 e = exp_of_token<T, N>(a.h, b, valid);
-  if (lane < kTokens) {
+  if (valid) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       *reinterpret_cast<float4*>(etile + 16 * lane + 4 * q) =
           make_float4(e.v[4 * q], e.v[4 * q + 1], e.v[4 * q + 2], e.v[4 * q + 3]);
-    if (a.aux && valid) {
+    if (a.aux && wave == 0) {
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -197,196 +228,235 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* etile = etile_mem[wave];
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves;
-  const int64_t span = static_cast<int64_t>(64) * V * kChunks;  // columns per pass
-  for (int64_t set = static_cast<int64_t>(blockIdx.x) * kWaves + wave; set < sets; set += stride) {
-    const TokenSet ts = token_set(set, sets, a.batch);
-    exp_tokens<T, N>(a, ts, lane, etile);
-    for (int i = 0; i < ts.count; ++i) {
-      const int64_t b = ts.token(i);
-      const M4 e = read_token(etile, i);
-      const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
-      for (int64_t c0 = 0; c0 < a.cols; c0 += span) {
-        U32x4 raw[kChunks][N];
+  const Share sh = share_of(a, wave);
+  // One token's offsets stay below 2^31 (the host checks the spans).
+  const int cols = static_cast<int>(a.cols);
+  const int xr_step = static_cast<int>(a.xr);
+  // One pass of columns of token i into raw: kChunks chunks from chunk m on.
+  U32x4 raw[kChunks][N];
+  auto load = [&](int i, int m) {
+    const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, sh.token(i) * a.xb, ((N - 1) * a.xr + a.cols) * es);
 #pragma unroll
-        for (int u = 0; u < kChunks; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
+    for (int u = 0; u < kChunks; ++u) {
+      const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
-          for (int k = 0; k < N; ++k)
-            raw[u][k] = c < a.cols ? load16(xs, static_cast<int32_t>((k * a.xr + c) * es)) : U32x4{0, 0, 0, 0};
-        }
+      for (int k = 0; k < N; ++k)
+        raw[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
+    }
+  };
+  exp_tokens<T, N>(a, sh, lane, wave, etile);
+  for (int i = sh.first; sh.holds(i); i += sh.abreast) {
+    const M4 e = read_token(etile, i);
+    const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, sh.token(i) * N * a.cols, N * a.cols * es);
+    for (int m = 0; sh.column(m, 64 * V) < cols; m += kChunks) {
+      load(i, m);
 #pragma unroll
-        for (int u = 0; u < kChunks; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
-          Vec<T> xv[N];
+      for (int u = 0; u < kChunks; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
+        Vec<T> xv[N];
 #pragma unroll
-          for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
+        for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
 #pragma unroll
-          for (int i2 = 0; i2 < N; ++i2) {
-            Vec<T> y;
+        for (int i2 = 0; i2 < N; ++i2) {
+          Vec<T> y;
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-              float acc = __builtin_fmaf(e.v[4 * i2], xv[0].f[v], 0.f);
+          for (int v = 0; v < V; ++v) {
+            float acc = __builtin_fmaf(e.v[4 * i2], xv[0].f[v], 0.f);
 #pragma unroll
-              for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
-              y.f[v] = acc;
-            }
-            if (c < a.cols) store16(pack<T>(y), ys, static_cast<int32_t>((i2 * a.cols + c) * es));
+            for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
+            y.f[v] = acc;
           }
+          if (c < cols) store16(pack<T>(y), ys, (i2 * cols + c) * es);
         }
       }
     }
-    lds_order();
   }
 }
 
-// Sum of 16 per-lane values over the wavefront, reduce-scatter style: after
-// exchanging halves with the lane 1, 2, 4, 8 apart (keeping the half this
-// lane's bit selects) every lane of a 16-lane row holds the row's sum of one
-// entry, entry = bit-reverse(lane & 15); two more exchanges (16, 32 apart) add
-// the rows.  Fixed order: every entry's sum is ((r0 + r1) + (r2 + r3)) of
-// fixed per-row trees.  Returns the total of entry bitrev4(lane & 15).
-__device__ __forceinline__ float wave_sum16(const float (&v)[16], int lane) {
-  float a[16];
+// Value of the lane whose index differs in bit 3 (row_ror:8) or bit 2
+// (row_ror:4 for lanes with the bit set, row_ror:12 for the others) or by a
+// permutation of the quad.
+template <int Quad>
+__device__ __forceinline__ float quad_lane(float v) {
+  const int w = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(w, w, Quad, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_xor8(float v) {
+  const int w = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(w, w, 0x128, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_xor4(float v) {
+  const int w = __float_as_int(v);
+  const int t = __builtin_amdgcn_update_dpp(w, w, 0x124, 0xF, 0xA, false);
+  return __int_as_float(__builtin_amdgcn_update_dpp(t, w, 0x12C, 0xF, 0x5, false));
+}
+
+// Sums of M per-lane values (a power of two up to 64) over the wavefront,
+// reduce-scatter style: six exchanges with the lane 32, 16, 8, 4, 2, 1 apart;
+// while more than one value is left, each keeps the half this lane's bit
+// selects.  Lane l returns the total of entry l / (64 / M), summed in a fixed
+// tree.  The first two exchanges are register swaps between halves and between
+// rows of the wavefront, the others DPP moves: against exchanges through
+// ds_bpermute the backward at 16384 x 2 x 4096 BF16 ran 189 -> 135 us and at 16384 x 4 x 1024 86 -> 79 us.
+template <int M>
+__device__ __forceinline__ float wave_sum(const float (&v)[M], int lane) {
+  float a[M];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) a[e] = v[e];
+  for (int e = 0; e < M; ++e) a[e] = v[e];
 #pragma unroll
-  for (int step = 0; step < 4; ++step) {
-    const int half = 8 >> step;
-    const bool upper = (lane >> step) & 1;
+  for (int step = 0; step < 6; ++step) {
+    const int half = M >> (step + 1);
+    const bool upper = (lane >> (5 - step)) & 1;
 #pragma unroll
-    for (int j = 0; j < half; ++j) {
-      const float keep = upper ? a[j + half] : a[j];
-      const float send = upper ? a[j] : a[j + half];
-      a[j] = keep + __shfl_xor(send, 1 << step);
+    for (int j = 0; j < (half > 0 ? half : 1); ++j) {
+      const float x = a[j];
+      const float y = half > 0 ? a[j + half] : a[j];
+      if (step < 2) {
+        // Swaps x of the upper lanes with y of the lower ones: the sum of both
+        // registers is x's pair sum in the lower lanes, y's in the upper.
+        typedef uint32_t U2 __attribute__((ext_vector_type(2)));
+        const U2 s = step == 0
+                         ? __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false)
+                         : __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        a[j] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+      } else {
+        const float keep = upper ? y : x;
+        const float send = upper ? x : y;
+        a[j] = keep + (step == 2   ? lane_xor8(send)
+                       : step == 3 ? lane_xor4(send)
+                       : step == 4 ? quad_lane<0x4E>(send)
+                                   : quad_lane<0xB1>(send));
+      }
     }
   }
-  float t = a[0] + __shfl_xor(a[0], 16);
-  return t + __shfl_xor(t, 32);
+  return a[0];
 }
-
-__device__ __forceinline__ int bitrev4(int x) { return ((x & 1) << 3) | ((x & 2) << 1) | ((x & 4) >> 1) | ((x & 8) >> 3); }
 
 // Backward: dX row k = sum_r E[r][k] dY[r] (fmaf chain r = 0..n-1 from +0);
 // dE[r][k] = sum_c dY[r][c] X[k][c] (per lane in column order, then
-// wave_sum16); dH = L(H^T, dE).
+// wave_sum, then the wavefronts' parts in order); dH = L(H^T, dE).
 template <typename T, int N>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_mix_bwd_kernel(HcArgs a) {
   __shared__ __attribute__((aligned(16))) float etile_mem[kWaves][kTokens * 16];
-  __shared__ __attribute__((aligned(16))) float gtile_mem[kWaves][kTokens * 16];
+  __shared__ __attribute__((aligned(16))) float gtile_mem[kWaves][kTokens * 16];  // dE by column part
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
   constexpr int V = Vec<T>::V;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* etile = etile_mem[wave];
-  float* gtile = gtile_mem[wave];
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves;
-  const int64_t span = static_cast<int64_t>(64) * V * kChunksBwd;
-  for (int64_t set = static_cast<int64_t>(blockIdx.x) * kWaves + wave; set < sets; set += stride) {
-    const TokenSet ts = token_set(set, sets, a.batch);
-    exp_tokens<T, N>(a, ts, lane, etile);
-    for (int i = 0; i < ts.count; ++i) {
-      const int64_t b = ts.token(i);
-      const M4 e = read_token(etile, i);
-      const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t gs = rebased<T>(a.gy, b * a.gb, ((N - 1) * a.gr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t ds = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
-      float acc[16];
+  const Share sh = share_of(a, wave);
+  // One token's offsets stay below 2^31 (the host checks the spans).
+  const int cols = static_cast<int>(a.cols);
+  const int xr_step = static_cast<int>(a.xr);
+  const int gr_step = static_cast<int>(a.gr);
+  exp_tokens<T, N>(a, sh, lane, wave, etile);
+  for (int i = sh.first; sh.holds(i); i += sh.abreast) {
+    const int64_t b = sh.token(i);
+    const M4 e = read_token(etile, i);
+    const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
+    const __amdgpu_buffer_rsrc_t gs = rebased<T>(a.gy, b * a.gb, ((N - 1) * a.gr + a.cols) * es);
+    const __amdgpu_buffer_rsrc_t ds = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
+    constexpr int M = N == 2 ? 4 : 16;  // entries r N + k of dE, a power of two
+    float acc[M];
 #pragma unroll
-      for (int q = 0; q < 16; ++q) acc[q] = 0.f;
-      for (int64_t c0 = 0; c0 < a.cols; c0 += span) {
-        U32x4 xr[kChunksBwd][N], gr[kChunksBwd][N];
+    for (int q = 0; q < M; ++q) acc[q] = 0.f;
+    for (int m = 0; sh.column(m, 64 * V) < cols; m += kChunksBwd) {
+      U32x4 xr[kChunksBwd][N], gr[kChunksBwd][N];
 #pragma unroll
-        for (int u = 0; u < kChunksBwd; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
+      for (int u = 0; u < kChunksBwd; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
-          for (int k = 0; k < N; ++k) {
-            xr[u][k] = c < a.cols ? load16(xs, static_cast<int32_t>((k * a.xr + c) * es)) : U32x4{0, 0, 0, 0};
-            gr[u][k] = c < a.cols ? load16(gs, static_cast<int32_t>((k * a.gr + c) * es)) : U32x4{0, 0, 0, 0};
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kChunksBwd; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
-          Vec<T> xv[N], gv[N];
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            xv[k] = unpack<T>(xr[u][k]);
-            gv[k] = unpack<T>(gr[u][k]);
-          }
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            Vec<T> dx;
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-              float d = __builtin_fmaf(e.v[k], gv[0].f[v], 0.f);
-#pragma unroll
-              for (int r = 1; r < N; ++r) d = __builtin_fmaf(e.v[4 * r + k], gv[r].f[v], d);
-              dx.f[v] = d;
-            }
-            if (c < a.cols) store16(pack<T>(dx), ds, static_cast<int32_t>((k * a.cols + c) * es));
-          }
-#pragma unroll
-          for (int r = 0; r < N; ++r)
-#pragma unroll
-            for (int k = 0; k < N; ++k)
-#pragma unroll
-              for (int v = 0; v < V; ++v) acc[4 * r + k] = __builtin_fmaf(gv[r].f[v], xv[k].f[v], acc[4 * r + k]);
+        for (int k = 0; k < N; ++k) {
+          xr[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
+          gr[u][k] = c < cols ? load16(gs, (k * gr_step + c) * es) : U32x4{0, 0, 0, 0};
         }
       }
-      const float total = wave_sum16(acc, lane);
-      if (lane < 16) gtile[16 * i + bitrev4(lane)] = total;
-    }
-    lds_order();
-    // L(H^T, dE) of the set's token lane % kTokens.
-    const int slot = lane & (kTokens - 1);
-    const int64_t b = ts.token(slot);
-    const bool valid = slot < ts.count;
-    PM<true> cur;
-    if (valid) {
-      const M4 h = load_elements<T>(a.h, b, N);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int u = 0; u < kChunksBwd; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
+        Vec<T> xv[N], gv[N];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) cur.d.v[4 * r + c] = h.v[4 * c + r];
-      cur.u = read_token(gtile, slot);
-      // The debug copy of dE goes out now, so that cur.u is not kept live
-      // across the Frechet polynomial (it would spill at the 256-VGPR cap).
-      if (a.aux && lane < kTokens) {
+        for (int k = 0; k < N; ++k) {
+          xv[k] = unpack<T>(xr[u][k]);
+          gv[k] = unpack<T>(gr[u][k]);
+        }
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          Vec<T> dx;
+#pragma unroll
+          for (int v = 0; v < V; ++v) {
+            float d = __builtin_fmaf(e.v[k], gv[0].f[v], 0.f);
+#pragma unroll
+            for (int r = 1; r < N; ++r) d = __builtin_fmaf(e.v[4 * r + k], gv[r].f[v], d);
+            dx.f[v] = d;
+          }
+          if (c < cols) store16(pack<T>(dx), ds, (k * cols + c) * es);
+        }
 #pragma unroll
         for (int r = 0; r < N; ++r)
 #pragma unroll
-          for (int k = 0; k < N; ++k) a.aux[b * N * N + r * N + k] = cur.u.v[4 * r + k];
-      }
-    } else {
+          for (int k = 0; k < N; ++k)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        cur.d.v[q] = 0.f;
-        cur.u.v[q] = 0.f;
+            for (int v = 0; v < V; ++v) acc[N * r + k] = __builtin_fmaf(gv[r].f[v], xv[k].f[v], acc[N * r + k]);
       }
     }
-    M4 dh;
-    const int s = expm_lane<true>(cur, a.h.sign, 1.f, [&](const M4& out) { dh = out; });
-    if (s < 0) {
-#pragma unroll
-      for (int q = 0; q < 16; ++q) dh.v[q] = __builtin_nanf("");
-    }
-    if (lane < kTokens && valid) store_elements<T>(a.dh, b, N, dh);
-    lds_order();
+    const float total = wave_sum(acc, lane);
+    const int entry = lane / (64 / M);
+    if (lane % (64 / M) == 0 && entry < N * N) gtile_mem[sh.part][16 * i + 4 * (entry / N) + entry % N] = total;
   }
+  __syncthreads();
+  if (wave != 0) return;
+  // L(H^T, dE) of the set's token `lane`.
+  const int64_t b = sh.token(lane);
+  const bool valid = sh.holds(lane);
+  PM<true> cur;
+  if (valid) {
+    const M4 h = load_elements<T>(a.h, b, N);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) cur.d.v[4 * r + c] = h.v[4 * c + r];
+    cur.u = read_token(gtile_mem[0], lane);
+    for (int p = 1; p < sh.parts; ++p) {
+      const M4 more = read_token(gtile_mem[p], lane);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) cur.u.v[q] += more.v[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      if (q / 4 >= N || q % 4 >= N) cur.u.v[q] = 0.f;
+    // The debug copy of dE goes out now, so that cur.u is not kept live
+    // across the Frechet polynomial (it would spill at the 256-VGPR cap).
+    if (a.aux) {
+#pragma unroll
+      for (int r = 0; r < N; ++r)
+#pragma unroll
+        for (int k = 0; k < N; ++k) a.aux[b * N * N + r * N + k] = cur.u.v[4 * r + k];
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      cur.d.v[q] = 0.f;
+      cur.u.v[q] = 0.f;
+    }
+  }
+  M4 dh;
+  const int s = expm_lane<true>(cur, a.h.sign, 1.f, [&](const M4& out) { dh = out; });
+  if (s < 0) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) dh.v[q] = __builtin_nanf("");
+  }
+  if (valid) store_elements<T>(a.dh, b, N, dh);
 }
 
 // ---- 5 <= n <= 8 streams: exp(H) supplied in FP32 ----------------------------
 //
 // For n = 5..8 the exponential runs in its own kernel (P = 8, FP32 output, the
 // same bits the fused path would keep on chip); these kernels apply it.  The
-// token sets, row streaming and nontemporal hints are the fused kernels'.
-// E of the set's tokens sits in LDS in rows of 8 floats (64 per token): E
-// itself for the forward, E^T for the backward, so that the row an output
-// row needs is two 16-byte broadcast reads.
+// token sets, column shares, row streaming and nontemporal hints are the fused
+// kernels'.  E of the set's tokens sits in the workgroup's LDS in rows of 8
+// floats (64 per token): E itself for the forward, E^T for the backward, so
+// that the row an output row needs is two 16-byte broadcast reads.
 
 struct WideArgs {
   const float* e;   // FP32 [B, n, n], contiguous
@@ -398,6 +468,9 @@ struct WideArgs {
   float* de;        // backward: dE = dY X^T, FP32 [B, n, n], contiguous
   int64_t batch;
   int64_t cols;
+  int64_t sets;     // workgroups
+  int tokens;       // per workgroup
+  int parts;        // wavefronts that share a token's columns (column_parts)
   int n;
 };
 
@@ -451,18 +524,27 @@ __device__ __forceinline__ void store8(U32x2 w, __amdgpu_buffer_rsrc_t rs, int32
   __builtin_amdgcn_raw_buffer_store_b64(w, rs, voff, 0, kStreamPolicy);
 }
 
-// E of the set's tokens into `etile` (64 floats per token, rows of 8): lane
-// 8 j + p copies row p of token j's E (transposed: column p) when both exist.
+// E of the set's tokens into `etile` (64 floats per token, rows of 8), eight
+// threads a token: thread p of them copies row p (transposed: column p).  The
+// whole workgroup loads the tokens its wavefronts share; when they share none,
+// each wavefront loads its own and waits for no other.
 template <int N, bool Transposed>
-__device__ __forceinline__ void load_set_e(const WideArgs& a, const TokenSet& ts, int lane, float* etile) {
-  const int j = lane >> 3;
-  const int p = lane & 7;
-  if (j < ts.count && p < N) {
-    const float* src = a.e + ts.token(j) * (N * N);
+__device__ __forceinline__ void load_set_e(const WideArgs& a, const Share& sh, int lane, float* etile) {
+  const bool shared = sh.parts > 1;
+  const int p = threadIdx.x & 7;
+  for (int t = (shared ? threadIdx.x : lane) >> 3; t < sh.slots; t += shared ? 8 * kWaves : 8) {
+    const int j = shared ? t : sh.first + t * sh.abreast;
+    if (p < N && sh.holds(j)) {
+      const float* src = a.e + sh.token(j) * (N * N);
 #pragma unroll
-    for (int k = 0; k < N; ++k) etile[64 * j + 8 * p + k] = Transposed ? src[k * N + p] : src[p * N + k];
+      for (int k = 0; k < N; ++k) etile[64 * j + 8 * p + k] = Transposed ? src[k * N + p] : src[p * N + k];
+    }
   }
-  lds_order();
+  if (shared) {
+    __syncthreads();
+  } else {
+    lds_order();
+  }
 }
 
 // Row r of the token's 8-float rows (the first N entries are used).
@@ -476,172 +558,163 @@ __device__ __forceinline__ void read_row8(const float* tile, int token, int r, f
 // Forward: row i of Y = sum_k E[i][k] X[k] (fmaf chain k = 0..n-1 from +0).
 template <typename T, int N>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_wide_fwd_kernel(WideArgs a) {
-  __shared__ __attribute__((aligned(16))) float etile_mem[kWaves][kTokens * 64];
+  __shared__ __attribute__((aligned(16))) float etile[kTokens * 64];
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
   constexpr int V = Vec<T>::V;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float* etile = etile_mem[wave];
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves;
-  const int64_t span = static_cast<int64_t>(64) * V * kWideChunks;
-  for (int64_t set = static_cast<int64_t>(blockIdx.x) * kWaves + wave; set < sets; set += stride) {
-    const TokenSet ts = token_set(set, sets, a.batch);
-    load_set_e<N, false>(a, ts, lane, etile);
-    for (int i = 0; i < ts.count; ++i) {
-      const int64_t b = ts.token(i);
-      float e[N][8];
+  const Share sh = share_of(a, wave);
+  // One token's offsets stay below 2^31 (the host checks the spans).
+  const int cols = static_cast<int>(a.cols);
+  const int xr_step = static_cast<int>(a.xr);
+  load_set_e<N, false>(a, sh, lane, etile);
+  for (int i = sh.first; sh.holds(i); i += sh.abreast) {
+    const int64_t b = sh.token(i);
+    float e[N][8];
 #pragma unroll
-      for (int r = 0; r < N; ++r) read_row8(etile, i, r, e[r]);
-      const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
-      for (int64_t c0 = 0; c0 < a.cols; c0 += span) {
-        U32x4 raw[kWideChunks][N];
+    for (int r = 0; r < N; ++r) read_row8(etile, i, r, e[r]);
+    const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
+    const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
+    for (int m = 0; sh.column(m, 64 * V) < cols; m += kWideChunks) {
+      U32x4 raw[kWideChunks][N];
 #pragma unroll
-        for (int u = 0; u < kWideChunks; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
+      for (int u = 0; u < kWideChunks; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
-          for (int k = 0; k < N; ++k)
-            raw[u][k] = c < a.cols ? load16(xs, static_cast<int32_t>((k * a.xr + c) * es)) : U32x4{0, 0, 0, 0};
-        }
+        for (int k = 0; k < N; ++k)
+          raw[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
+      }
 #pragma unroll
-        for (int u = 0; u < kWideChunks; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
-          Vec<T> xv[N];
+      for (int u = 0; u < kWideChunks; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
+        Vec<T> xv[N];
 #pragma unroll
-          for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
+        for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
 #pragma unroll
-          for (int i2 = 0; i2 < N; ++i2) {
-            Vec<T> y;
+        for (int i2 = 0; i2 < N; ++i2) {
+          Vec<T> y;
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-              float acc = __builtin_fmaf(e[i2][0], xv[0].f[v], 0.f);
+          for (int v = 0; v < V; ++v) {
+            float acc = __builtin_fmaf(e[i2][0], xv[0].f[v], 0.f);
 #pragma unroll
-              for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e[i2][k], xv[k].f[v], acc);
-              y.f[v] = acc;
-            }
-            if (c < a.cols) store16(pack<T>(y), ys, static_cast<int32_t>((i2 * a.cols + c) * es));
+            for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e[i2][k], xv[k].f[v], acc);
+            y.f[v] = acc;
           }
+          if (c < cols) store16(pack<T>(y), ys, (i2 * cols + c) * es);
         }
       }
     }
-    lds_order();
   }
-}
-
-// Sum of 64 per-lane values over the wavefront, reduce-scatter style: six
-// exchanges with the lane 1, 2, 4, 8, 16, 32 apart, each keeping the half
-// this lane's bit selects, leave every lane with the total of one entry,
-// entry = bit-reverse(lane) (6 bits), summed in a fixed tree.
-__device__ __forceinline__ float wave_sum64(const float (&v)[64], int lane) {
-  float a[64];
-#pragma unroll
-  for (int e = 0; e < 64; ++e) a[e] = v[e];
-#pragma unroll
-  for (int step = 0; step < 6; ++step) {
-    const int half = 32 >> step;
-    const bool upper = (lane >> step) & 1;
-#pragma unroll
-    for (int j = 0; j < half; ++j) {
-      const float keep = upper ? a[j + half] : a[j];
-      const float send = upper ? a[j] : a[j + half];
-      a[j] = keep + __shfl_xor(send, 1 << step);
-    }
-  }
-  return a[0];
-}
-
-__device__ __forceinline__ int bitrev6(int x) {
-  return ((x & 1) << 5) | ((x & 2) << 3) | ((x & 4) << 1) | ((x & 8) >> 1) | ((x & 16) >> 3) | ((x & 32) >> 5);
 }
 
 // Backward: dX row k = sum_r E[r][k] dY[r] (fmaf chain r = 0..n-1 from +0);
 // dE[r][k] = sum_c dY[r][c] X[k][c] (per lane in column order, then
-// wave_sum64), written to a.de.
+// wave_sum, then the wavefronts' parts in order), written to a.de.
 template <typename T, int N>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_wide_bwd_kernel(WideArgs a) {
-  __shared__ __attribute__((aligned(16))) float etile_mem[kWaves][kTokens * 64];
+  __shared__ __attribute__((aligned(16))) float etile[kTokens * 64];
+  __shared__ float gtile[kWaves][kTokens * 64];  // dE by column part
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
   constexpr int V = Vec8<T>::V;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float* etile = etile_mem[wave];
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves;
-  const int64_t span = static_cast<int64_t>(64) * V * kWideChunksBwd;
-  const int entry = bitrev6(lane);
-  for (int64_t set = static_cast<int64_t>(blockIdx.x) * kWaves + wave; set < sets; set += stride) {
-    const TokenSet ts = token_set(set, sets, a.batch);
-    load_set_e<N, true>(a, ts, lane, etile);
-    for (int i = 0; i < ts.count; ++i) {
-      const int64_t b = ts.token(i);
-      const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t gs = rebased<T>(a.gy, b * a.gb, ((N - 1) * a.gr + a.cols) * es);
-      const __amdgpu_buffer_rsrc_t ds = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
-      float acc[64];
+  const Share sh = share_of(a, wave);
+  // One token's offsets stay below 2^31 (the host checks the spans).
+  const int cols = static_cast<int>(a.cols);
+  const int xr_step = static_cast<int>(a.xr);
+  const int gr_step = static_cast<int>(a.gr);
+  load_set_e<N, true>(a, sh, lane, etile);
+  for (int i = sh.first; sh.holds(i); i += sh.abreast) {
+    const int64_t b = sh.token(i);
+    const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
+    const __amdgpu_buffer_rsrc_t gs = rebased<T>(a.gy, b * a.gb, ((N - 1) * a.gr + a.cols) * es);
+    const __amdgpu_buffer_rsrc_t ds = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
+    float acc[64];
 #pragma unroll
-      for (int q = 0; q < 64; ++q) acc[q] = 0.f;
-      for (int64_t c0 = 0; c0 < a.cols; c0 += span) {
-        U32x2 xr[kWideChunksBwd][N], gr[kWideChunksBwd][N];
+    for (int q = 0; q < 64; ++q) acc[q] = 0.f;
+    for (int m = 0; sh.column(m, 64 * V) < cols; m += kWideChunksBwd) {
+      U32x2 xr[kWideChunksBwd][N], gr[kWideChunksBwd][N];
 #pragma unroll
-        for (int u = 0; u < kWideChunksBwd; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
+      for (int u = 0; u < kWideChunksBwd; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
-          for (int k = 0; k < N; ++k) {
-            xr[u][k] = c < a.cols ? load8(xs, static_cast<int32_t>((k * a.xr + c) * es)) : U32x2{0, 0};
-            gr[u][k] = c < a.cols ? load8(gs, static_cast<int32_t>((k * a.gr + c) * es)) : U32x2{0, 0};
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kWideChunksBwd; ++u) {
-          const int64_t c = c0 + (u * 64 + lane) * V;
-          Vec8<T> xv[N], gv[N];
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            xv[k] = unpack8<T>(xr[u][k]);
-            gv[k] = unpack8<T>(gr[u][k]);
-          }
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            float col[8];
-            read_row8(etile, i, k, col);  // column k of E
-            Vec8<T> dx;
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-              float d = __builtin_fmaf(col[0], gv[0].f[v], 0.f);
-#pragma unroll
-              for (int r = 1; r < N; ++r) d = __builtin_fmaf(col[r], gv[r].f[v], d);
-              dx.f[v] = d;
-            }
-            if (c < a.cols) store8(pack8<T>(dx), ds, static_cast<int32_t>((k * a.cols + c) * es));
-          }
-#pragma unroll
-          for (int r = 0; r < N; ++r)
-#pragma unroll
-            for (int k = 0; k < N; ++k)
-#pragma unroll
-              for (int v = 0; v < V; ++v) acc[r * N + k] = __builtin_fmaf(gv[r].f[v], xv[k].f[v], acc[r * N + k]);
+        for (int k = 0; k < N; ++k) {
+          xr[u][k] = c < cols ? load8(xs, (k * xr_step + c) * es) : U32x2{0, 0};
+          gr[u][k] = c < cols ? load8(gs, (k * gr_step + c) * es) : U32x2{0, 0};
         }
       }
-      const float total = wave_sum64(acc, lane);
-      if (entry < N * N) a.de[b * (N * N) + entry] = total;
+#pragma unroll
+      for (int u = 0; u < kWideChunksBwd; ++u) {
+        const int c = sh.column(m + u, 64 * V) + lane * V;
+        Vec8<T> xv[N], gv[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          xv[k] = unpack8<T>(xr[u][k]);
+          gv[k] = unpack8<T>(gr[u][k]);
+        }
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+          float col[8];
+          read_row8(etile, i, k, col);  // column k of E
+          Vec8<T> dx;
+#pragma unroll
+          for (int v = 0; v < V; ++v) {
+            float d = __builtin_fmaf(col[0], gv[0].f[v], 0.f);
+#pragma unroll
+            for (int r = 1; r < N; ++r) d = __builtin_fmaf(col[r], gv[r].f[v], d);
+            dx.f[v] = d;
+          }
+          if (c < cols) store8(pack8<T>(dx), ds, (k * cols + c) * es);
+        }
+#pragma unroll
+        for (int r = 0; r < N; ++r)
+#pragma unroll
+          for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[r * N + k] = __builtin_fmaf(gv[r].f[v], xv[k].f[v], acc[r * N + k]);
+      }
     }
-    lds_order();
+    const float total = wave_sum(acc, lane);
+    if (sh.parts == 1) {
+      if (lane < N * N) a.de[b * (N * N) + lane] = total;
+    } else {
+      gtile[sh.part][64 * i + lane] = total;
+    }
+  }
+  if (sh.parts == 1) return;
+  __syncthreads();
+  for (int t = threadIdx.x; t < 64 * sh.slots; t += 64 * kWaves) {
+    const int entry = t & 63;
+    if (entry < N * N && sh.holds(t >> 6)) {
+      float total = gtile[0][t];
+      for (int p = 1; p < sh.parts; ++p) total += gtile[p][t];
+      a.de[sh.token(t >> 6) * (N * N) + entry] = total;
+    }
   }
 }
 
-// Grid: one wavefront per token set up to what the device keeps resident
-// (counted once per kernel; the wavefronts stride over the rest).
-template <typename T, int N, bool Backward>
-hipError_t launch_one(const HcArgs& a, hipStream_t stream) {
-  const auto kernel = Backward ? hc_mix_bwd_kernel<T, N> : hc_mix_fwd_kernel<T, N>;
-  static const int64_t resident = resident_blocks(reinterpret_cast<const void*>(kernel), 64 * kWaves);
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  int64_t grid = (sets + kWaves - 1) / kWaves;
-  if (grid > resident) grid = resident;
-  if (grid < 1) grid = 1;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
+// Grid: two workgroups a compute unit, until each has `most` tokens; from there
+// on more workgroups, which the hardware starts as others retire (finer sets
+// balance the last ones, coarser sets pay for fewer exponentials).
+template <typename Args>
+hipError_t launch_sets(void (*kernel)(Args), Args a, int most, hipStream_t stream) {
+  static const int64_t target = 2 * compute_units();
+  const int abreast = kWaves / a.parts;
+  const int64_t rounds = (a.batch + target * abreast - 1) / (target * abreast);
+  a.tokens = rounds * abreast < most ? static_cast<int>(rounds * abreast) : most;
+  a.sets = (a.batch + a.tokens - 1) / a.tokens;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.sets)), dim3(64 * kWaves), 0, stream, a);
   return hipGetLastError();
+}
+
+// Largest sets, BF16, 40000 x 4 x 1024 and 16384 x 4 x 1024, us: forward
+// 8 / 16 / 32 tokens 112 / 116 / 122 and 49.5 / 49.8 / 49.7; backward, which
+// has a Frechet polynomial a set as well, 195 / 178 / 183 and 87 / 81 / 79.
+template <typename T, int N, bool Backward>
+hipError_t launch_one(HcArgs a, hipStream_t stream) {
+  const auto kernel = Backward ? hc_mix_bwd_kernel<T, N> : hc_mix_fwd_kernel<T, N>;
+  a.parts = column_parts(a.cols, 64 * Vec<T>::V * kChunksBwd);
+  return launch_sets(kernel, a, Backward ? kTokens : kTokens / 2, stream);
 }
 
 template <typename T>
@@ -656,16 +729,16 @@ hipError_t launch_t(const HcArgs& a, bool backward, hipStream_t stream) {
   }
 }
 
+// n = 5..8, the same at 16384 x 6 x 1024 and 16384 x 8 x 512: forward 8 / 16
+// tokens 68.7 / 70.6 and 47.3 / 46.4 us; backward 103 / 108 and, where a
+// wavefront has a single pass of a token, 83 / 80 us.
 template <typename T, int N, bool Backward>
-hipError_t launch_wide_one(const WideArgs& a, hipStream_t stream) {
+hipError_t launch_wide_one(WideArgs a, hipStream_t stream) {
   const auto kernel = Backward ? hc_wide_bwd_kernel<T, N> : hc_wide_fwd_kernel<T, N>;
-  static const int64_t resident = resident_blocks(reinterpret_cast<const void*>(kernel), 64 * kWaves);
-  const int64_t sets = (a.batch + kTokens - 1) / kTokens;
-  int64_t grid = (sets + kWaves - 1) / kWaves;
-  if (grid > resident) grid = resident;
-  if (grid < 1) grid = 1;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
-  return hipGetLastError();
+  constexpr int pass = 64 * (Backward ? Vec8<T>::V * kWideChunksBwd : Vec<T>::V * kWideChunks);
+  // The backward's reduction of 64 sums costs a fifth of a pass: two passes per wavefront at least.
+  a.parts = column_parts(a.cols, Backward ? 2 * pass : pass);
+  return launch_sets(kernel, a, Backward && a.cols <= pass ? kTokens : kTokens / 2, stream);
 }
 
 template <typename T, bool Backward>
@@ -684,8 +757,24 @@ hipError_t launch_wide_t(const WideArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// A launch takes at most kSlice tokens (a grid holds fewer than 2^24 workgroups
+// of 256 threads); a larger batch goes in slices.
+constexpr int64_t kSlice = int64_t{1} << 26;
+
+const void* advanced(const void* p, int64_t bytes) { return p ? static_cast<const char*>(p) + bytes : nullptr; }
+void* advanced(void* p, int64_t bytes) { return p ? static_cast<char*>(p) + bytes : nullptr; }
+
 hipError_t launch_hc_apply(const float* e, const void* x, const int64_t* xs, const void* gy, const int64_t* gs,
                            void* out, float* de, int dtype, int64_t batch, int n, int64_t cols, hipStream_t stream) {
+  if (batch > kSlice) {
+    const int64_t es = dtype == F32::code ? 4 : 2;
+    const hipError_t err = launch_hc_apply(e, x, xs, gy, gs, out, de, dtype, kSlice, n, cols, stream);
+    if (err != hipSuccess) return err;
+    return launch_hc_apply(e + kSlice * n * n, advanced(x, kSlice * xs[0] * es), xs,
+                           gy ? advanced(gy, kSlice * gs[0] * es) : nullptr, gs,
+                           advanced(out, kSlice * n * cols * es), de ? de + kSlice * n * n : nullptr, dtype,
+                           batch - kSlice, n, cols, stream);
+  }
   WideArgs a;
   a.e = e;
   a.x = x;
@@ -712,6 +801,16 @@ hipError_t launch_hc_apply(const float* e, const void* x, const int64_t* xs, con
 hipError_t launch_hc_mix(const Operand& h, const void* x, const int64_t* xs, const void* gy, const int64_t* gs,
                          void* out, void* dh, float* aux, int dtype, int64_t batch, int n, int64_t cols,
                          hipStream_t stream) {
+  if (batch > kSlice) {
+    const int64_t es = dtype == F32::code ? 4 : 2;
+    const hipError_t err = launch_hc_mix(h, x, xs, gy, gs, out, dh, aux, dtype, kSlice, n, cols, stream);
+    if (err != hipSuccess) return err;
+    Operand rest = h;
+    rest.data = advanced(h.data, kSlice * h.sb * es);
+    return launch_hc_mix(rest, advanced(x, kSlice * xs[0] * es), xs, gy ? advanced(gy, kSlice * gs[0] * es) : nullptr,
+                         gs, advanced(out, kSlice * n * cols * es), advanced(dh, kSlice * n * n * es),
+                         aux ? aux + kSlice * n * n : nullptr, dtype, batch - kSlice, n, cols, stream);
+  }
   HcArgs a;
   a.h = h;
   a.x = x;
