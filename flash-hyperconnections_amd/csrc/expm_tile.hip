@@ -1,6 +1,8 @@
 // P in {16, 32} kernel (n = 9..32): one 64-lane wavefront per matrix, every
-// product on FP32 MFMA (v_mfma_f32_16x16x4_f32 for P = 16,
-// v_mfma_f32_32x32x2_f32 for P = 32).
+// product on the matrix cores: P = 16 on v_mfma_f32_16x16x4_f32, P = 32 on
+// v_mfma_f32_32x32x16_bf16 with each FP32 value as the sum of three bf16 ones
+// (and on v_mfma_f32_32x32x2_f32 where that sum would not hold; the section on
+// bf16 below).
 //
 // Layout: a P x P matrix occupies R = P*P/64 VGPRs per lane in the MFMA
 // accumulator ("D") layout: lane l, VGPR r holds M[row(l, r)][l % P] with
@@ -36,9 +38,10 @@
 //   step together with the D chain (two independent MFMA chains, and each
 //   operand register dies after its step).
 // Each FP32 MFMA step equals an fmaf chain over its k terms in ascending
-// order, so results differ from the reference's sequential FMA chains only
-// through the order of the k terms within a product and that one U chain
-// (parity is by tolerance; s is bit-identical).
+// order, so at P = 16 results differ from the reference's sequential FMA chains
+// only through the order of the k terms within a product and that one U chain;
+// at P = 32 the bf16 sums round less often (parity is by tolerance; s is
+// bit-identical).
 #include "fh_kernels.h"
 
 namespace fh {
@@ -83,6 +86,14 @@ struct TileCfg<32> {
 template <int P>
 using Acc = typename TileCfg<P>::acc_t;
 
+// The lane's number, formed anew at each call so that nothing derived from an
+// earlier one is kept live: the P = 32 kernels have no registers to spare.
+__device__ __forceinline__ int fresh_lane() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
+
 template <int P>
 struct Tm {
   float v[TileCfg<P>::R];
@@ -95,26 +106,11 @@ struct PTm {
 };
 
 template <int P>
-__device__ __forceinline__ Acc<P> to_acc(const Tm<P>& m) {
-  Acc<P> a;
-#pragma unroll
-  for (int r = 0; r < TileCfg<P>::R; ++r) a[r] = m.v[r];
-  return a;
-}
-template <int P>
 __device__ __forceinline__ Tm<P> from_acc(const Acc<P>& a) {
   Tm<P> m;
 #pragma unroll
   for (int r = 0; r < TileCfg<P>::R; ++r) m.v[r] = a[r];
   return m;
-}
-
-// acc + X.Y, X given as X^T in the D layout.
-template <int P>
-__device__ __forceinline__ Acc<P> mma(const Tm<P>& xt, const Tm<P>& y, Acc<P> acc) {
-#pragma unroll
-  for (int r = 0; r < TileCfg<P>::R; ++r) acc = TileCfg<P>::mfma(xt.v[r], y.v[r], acc);
-  return acc;
 }
 
 // (D1, U1).(D2, U2) = (D1.D2, D1.U2 + U1.D2).  Step r feeds all three
@@ -171,7 +167,16 @@ __device__ __forceinline__ Tm<P> tile_read_transposed(const float* buf, int lane
   return t;
 }
 
-// D layout of M -> D layout of M^T (both halves of a pair in one round).
+// D layout of M -> D layout of M^T.
+template <int P>
+__device__ __forceinline__ Tm<P> transpose(const Tm<P>& a, float* buf, int lane) {
+  tile_write<P>(a, buf, lane);
+  lds_order();
+  const Tm<P> t = tile_read_transposed<P>(buf, lane);
+  lds_order();
+  return t;
+}
+// The same of both halves of a pair in one round.
 template <int P, bool Pair>
 __device__ __forceinline__ PTm<P, Pair> ptranspose(const PTm<P, Pair>& a, float* buf, int lane) {
   constexpr int T = P * (P + 1);
@@ -184,6 +189,219 @@ __device__ __forceinline__ PTm<P, Pair> ptranspose(const PTm<P, Pair>& a, float*
   lds_order();
   return t;
 }
+
+// ---- P = 32: products on the bf16 matrix instructions ---------------------------
+//
+// An FP32 value is the exact sum of three bf16 values, v = h + m + l with
+// |m| <= 2^-8 |v| and |l| <= 2^-16 |v|, and X.Y is the six products
+//   xh.yh + (xm.yh + xh.ym) + (xl.yh + xm.ym + xh.yl)
+// (the three left out are below 2^-24 |x||y|), summed smallest first in one
+// FP32 accumulator.  Products of bf16 values are exact and an instruction sums 16
+// of them before it rounds, so the result is closer to the exact product than the
+// FP32 instructions' chain: over 512 products of N(0, 1) matrices 3.8e-8 against
+// 1.03e-7 relative error in the 2-norm (cutting values instead of rounding them
+// to their parts gave that advantage away over a whole exponential).
+//
+// Six bf16 instructions take 3/8 of the FP32 ones' cycles; splitting a matrix
+// costs 16 conversions, shifts or masks and subtractions a lane and part.
+// 32768 32 x 32 FP16 matrices, norms over 1.8 decades, forward + Frechet:
+// 577 -> 409 us (288 + 1061 -> 190 + 622 thousand cycles; the chip runs this
+// kernel at 1.9 GHz, the FP32 one at 2.3).  P = 16 keeps the FP32 instructions:
+// its products are shorter against the splits (341 -> 329 thousand cycles, at the
+// lower clock 150 -> 170 us over 65536 matrices).
+//
+// The k index is permuted as for the FP32 instructions: the B operand of Y
+// comes from the lane's own D-layout values, eight to a 32x32x16 instruction.
+// The A operand is the transposed X: its parts go to LDS column by column (8
+// bytes, four rows, to a write) and come back through the transposing read
+// ds_read_b64_tr_b16, which hands lane i of a row of 16 element i of each of four
+// columns.  So a matrix is split once for both sides.
+
+typedef __bf16 Bf16x8 __attribute__((ext_vector_type(8)));
+typedef short Short4 __attribute__((ext_vector_type(4)));
+typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
+
+// Parts of a matrix: w[k][s] holds part k of VGPRs 8s..8s+7, two to a word.  N of
+// the three parts are non-zero: BF16 inputs have one, FP16 inputs (11 bits) two.
+template <int N>
+struct Parts {
+  U32x4 w[N][2];
+};
+template <bool Pair, int N = 3>
+struct PParts {
+  Parts<N> d, u;
+};
+template <typename T>
+constexpr int kInputParts = T::code == F32::code ? 3 : T::code == F16::code ? 2 : 1;
+
+// (bf16(lo), bf16(hi)) in one word, round to nearest even.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef float Float2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((Float2{lo, hi}), Bf16x2));
+}
+
+template <int N>
+__device__ __forceinline__ Parts<N> split(const Tm<32>& m) {
+  // The mask in a VGPR: an SGPR operand costs a full-rate instruction 1.5x.
+  uint32_t mask;
+  asm("v_mov_b32 %0, 0xffff0000" : "=v"(mask));
+  Parts<N> p;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float a = m.v[2 * i], b = m.v[2 * i + 1];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const uint32_t w = pack_bf16(a, b);
+      p.w[k][i / 4][i % 4] = w;
+      a -= __uint_as_float(w << 16);
+      b -= __uint_as_float(w & mask);
+    }
+  }
+  return p;
+}
+template <int N, bool Pair>
+__device__ __forceinline__ PParts<Pair, N> psplit(const PTm<32, Pair>& m) {
+  PParts<Pair, N> p;
+  p.d = split<N>(m.d);
+  if constexpr (Pair) p.u = split<N>(m.u);
+  return p;
+}
+
+// LDS image of one part: column by column, its rows in chunks of four (8 bytes);
+// lane group g's VGPRs 4q..4q+3 are chunk 2q + g of its column.  A lane writes the
+// chunks of its own column and reads back, per q, the lane's row of four columns.
+// Columns are 72 bytes apart: writes are free of bank conflicts, reads all but.
+constexpr int kPartPitch = 72;
+constexpr int kPartBytes = 32 * kPartPitch;
+struct PartLds {
+  char *wr, *rd;  // q = 0; 16 and 8 * kPartPitch bytes on per q
+  __device__ __forceinline__ PartLds(char* buf, int lane) {
+    const int g = lane >> 5, i = lane & 15;
+    wr = buf + (lane & 31) * kPartPitch + 8 * g;
+    rd = buf + (4 * g + (i >> 2)) * kPartPitch + 8 * ((i & 3) + ((lane & 16) >> 2));
+  }
+};
+
+// Transposed parts of a left operand, laid out as Parts are.
+template <int N>
+struct Left {
+  Parts<N> p;
+  __device__ __forceinline__ void through_lds(const Parts<N>& m, const PartLds& at, int slot) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<U32x2*>(at.wr + (3 * slot + k) * kPartBytes + 16 * q) =
+            U32x2{m.w[k][q / 2][2 * (q % 2)], m.w[k][q / 2][2 * (q % 2) + 1]};
+    lds_order();
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        using LdsShort4 = __attribute__((address_space(3))) Short4;
+        const U32x2 t = __builtin_bit_cast(
+            U32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (LdsShort4*)(at.rd + (3 * slot + k) * kPartBytes + 8 * kPartPitch * q)));
+        p.w[k][q / 2][2 * (q % 2)] = t[0];
+        p.w[k][q / 2][2 * (q % 2) + 1] = t[1];
+      }
+  }
+};
+template <bool Pair, int N>
+struct PLeft {
+  Left<N> d, u;
+};
+
+// Splits m into right operands y and, through LDS, the left ones; the second
+// half's split covers the first one's way through LDS.
+template <int N, bool Pair>
+__device__ __forceinline__ PLeft<Pair, N> to_left(const PTm<32, Pair>& m, PParts<Pair, N>& y, const PartLds& at) {
+  PLeft<Pair, N> x;
+  y.d = split<N>(m.d);
+  x.d.through_lds(y.d, at, 0);
+  if constexpr (Pair) {
+    y.u = split<N>(m.u);
+    x.u.through_lds(y.u, at, 1);
+  }
+  lds_order();
+  return x;
+}
+
+// acc + the products of parts i of x and j of y with Lo <= i + j <= Hi, smallest
+// first.
+template <int Hi, int Lo, int NX, int NY>
+__device__ __forceinline__ v16f madd(const Left<NX>& x, const Parts<NY>& y, v16f acc) {
+#pragma unroll
+  for (int t = Hi; t >= Lo; --t)
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int j = t - i;
+      if (j < 0 || j >= NY) continue;
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(Bf16x8, x.p.w[i][s]),
+                                                      __builtin_bit_cast(Bf16x8, y.w[j][s]), acc, 0, 0, 0);
+    }
+  return acc;
+}
+
+// pmm on the bf16 instructions.  Every chain takes its small products first, so
+// that only the last few instructions round at the result's magnitude.
+template <bool Pair, bool WantD = true, int NX, int NY>
+__device__ __forceinline__ PTm<32, Pair> split_pmm(const PLeft<Pair, NX>& x, const PParts<Pair, NY>& y) {
+  v16f d = {}, u = {};
+  if constexpr (WantD) d = madd<2, 1>(x.d, y.d, d);
+  if constexpr (Pair) {
+    u = madd<2, 1>(x.d, y.u, u);
+    u = madd<2, 1>(x.u, y.d, u);
+  }
+  if constexpr (WantD) d = madd<0, 0>(x.d, y.d, d);
+  if constexpr (Pair) {
+    u = madd<0, 0>(x.d, y.u, u);
+    u = madd<0, 0>(x.u, y.d, u);
+  }
+  PTm<32, Pair> out;
+  out.d = from_acc<32>(d);
+  if constexpr (Pair) out.u = from_acc<32>(u);
+  return out;
+}
+
+// bf16 MFMAs read subnormal operands as zero.  The parts of v keep its bits while
+// |v| is 0 or at least 2^-100; matrices with smaller entries (scaled by 2^-s)
+// take the FP32 instructions.  FP16 inputs cannot have any: s <= 22.
+template <typename T, bool Pair>
+__device__ __forceinline__ bool splittable(const PTm<32, Pair>& a) {
+  if constexpr (T::code == F16::code) return true;
+  constexpr uint32_t kLeast = ((127u - 100u) << 24) - 1u;
+  // Twice the magnitude's bits minus one: zero becomes the largest value.
+  uint32_t least = ~0u;
+#pragma unroll
+  for (int r = 0; r < TileCfg<32>::R; ++r) {
+    least = min(least, (__float_as_uint(a.d.v[r]) << 1) - 1u);
+    if constexpr (Pair) least = min(least, (__float_as_uint(a.u.v[r]) << 1) - 1u);
+  }
+  return __builtin_amdgcn_ballot_w64(least < kLeast) == 0;
+}
+
+// Whether squaring `m` keeps every partial product and sum finite (64 terms
+// below 2^120); otherwise a low part's product could overflow to the opposite
+// infinity and make NaN of a result that is infinite.
+template <bool Pair>
+__device__ __forceinline__ bool squares_in_range(const PTm<32, Pair>& m) {
+  float top = 0.f;
+#pragma unroll
+  for (int r = 0; r < TileCfg<32>::R; ++r) {
+    top = __builtin_fmaxf(top, __builtin_fabsf(m.d.v[r]));
+    if constexpr (Pair) top = __builtin_fmaxf(top, __builtin_fabsf(m.u.v[r]));
+  }
+  return __builtin_amdgcn_ballot_w64(!(top < 0x1p60f)) == 0;
+}
+
+// The polynomial has norm at most exp(theta18) = e^3.01 and i squarings raise
+// that to exp(theta18 2^i): four rounds (operands to e^24, results to e^48) need
+// no check.
+constexpr int kUncheckedSquarings = 4;
 
 // c0*I in the D layout for the two combines with an identity term (B3 and B4,
 // reference csrc/MatrixExpSmall.cuh:268-281), from `dreg`, the VGPR of this
@@ -266,7 +484,8 @@ constexpr int kLoadCols = 1;
 
 // Byte addressing of one operand in the D layout of the loaded matrix: the
 // matrix base goes into the descriptor, `lane_off` is this lane's offset for
-// VGPR 0 and step(r) * `major` the uniform offset of VGPR r.
+// VGPR 0 and step(r) * `major` the uniform offset of VGPR r; `major` is the
+// elements per D-layout row step, given by the caller (op.sc or op.sr).
 struct TileSrc {
   const char* data;
   int64_t sb;        // bytes per batch step
@@ -276,10 +495,9 @@ struct TileSrc {
 };
 
 template <typename T, int P>
-__device__ __forceinline__ TileSrc make_src(const Operand& op, int layout, int n, int lane) {
+__device__ __forceinline__ TileSrc make_src(const Operand& op, int layout, int64_t major, int n, int lane) {
   using C = TileCfg<P>;
   constexpr int es = ElemIO<T>::bytes;
-  const int64_t major = layout == kLoadCols ? op.sc : op.sr;
   const int64_t minor = layout == kLoadCols ? op.sr : op.sc;
   TileSrc s;
   s.data = static_cast<const char*>(op.data);
@@ -334,7 +552,7 @@ __device__ __forceinline__ void store_tile(void* out, int64_t b, int n, int lane
   const int32_t lane_off = (C::row0(lane) * n + C::col(lane)) * es;
   if constexpr (Full) {
 #pragma unroll
-    for (int r = 0; r < C::R; ++r) ElemIO<T>::template store<kNontemporal>(m.v[r], rs, lane_off + C::step(r) * P * es, 0);
+    for (int r = 0; r < C::R; ++r) ElemIO<T>::template store<kNontemporal>(m.v[r], rs, lane_off, C::step(r) * P * es);
   } else {
     const bool col_ok = C::col(lane) < n;
 #pragma unroll
@@ -367,8 +585,15 @@ __device__ __forceinline__ float norm_estimate(const PTm<P, Pair>& a) {
     p += __builtin_fabsf(a.d.v[r]);
     if constexpr (Pair) p += __builtin_fabsf(a.u.v[r]);
   }
-  if constexpr (P == 16) p += __shfl_xor(p, 16);
-  p += __shfl_xor(p, 32);
+  // Rows of 16 (P = 16) and halves of 32 exchanged in registers.
+  const uint32_t w = __float_as_uint(p);
+  if constexpr (P == 16) {
+    const auto rows = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    p = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+  }
+  const uint32_t v = __float_as_uint(p);
+  const auto halves = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  p = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
   uint32_t m = row_max_u32(__float_as_uint(p) & 0x7FFFFFFFu);
   uint32_t top = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m), 0));
   if constexpr (P == 32) top = max(top, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m), 16)));
@@ -417,52 +642,100 @@ constexpr int kTileWaves() {
   return P == 16 ? 4 : (Pair ? 2 : 3);
 }
 
+// LDS of a workgroup; P = 32 uses it for the FP32 transposes and the bf16 parts in
+// turn.
+template <int P, bool Pair>
+constexpr int kTileLds = (Pair ? 2 : 1) * (P == 32 ? 3 * kPartBytes : 4 * P * (P + 1));
+static_assert(3 * kPartBytes >= 4 * 32 * 33);
+
+// Degree-18 polynomial (csrc/MatrixExpSmall.cuh:83-106): A^2 = A.A,
+// A^3 = A.A^2, A^6 = A^3.A^3, A9 = B1.B5 + B4, T = B2 + (B3 + A9).A9.
+// The sums B1.B5 + B4, B3 + A9 and B2 + (..).A9 are formed after their
+// products, as in the reference: starting the MFMA accumulations from B4
+// and B2 instead raised the FP32 error 1.4-fold on average (measured over
+// 32768 32 x 32 matrices against the FP64 result and the reference's own
+// arithmetic).
+//
+// On the FP32 instructions; `at` is a's transpose and `lane()` the lane.
+template <int P, bool Pair, typename Lane>
+__device__ __forceinline__ PTm<P, Pair> polynomial(const PTm<P, Pair>& a, const PTm<P, Pair>& at, const Ident<P>& id,
+                                                   float* buf, Lane lane) {
+  const PTm<P, Pair> a2 = pmm<P, Pair>(at, a);
+  const PTm<P, Pair> a3 = pmm<P, Pair>(at, a2);
+  const PTm<P, Pair> a6 = pmm<P, Pair>(ptranspose<P, Pair>(a3, buf, lane()), a3);
+  const PTm<P, Pair> b1t = ptranspose<P, Pair>(combine<0, P, Pair>(a, a2, a3, a6, id), buf, lane());
+  const PTm<P, Pair> b5 = combine<4, P, Pair>(a, a2, a3, a6, id);
+  const PTm<P, Pair> b1b5 = pmm<P, Pair>(b1t, b5);
+  const PTm<P, Pair> a9 = padd<P, Pair>(b1b5, combine<3, P, Pair>(a, a2, a3, a6, id));
+  const PTm<P, Pair> lhst =
+      ptranspose<P, Pair>(padd<P, Pair>(combine<2, P, Pair>(a, a2, a3, a6, id), a9), buf, lane());
+  const PTm<P, Pair> b2 = combine<1, P, Pair>(a, a2, a3, a6, id);
+  return padd<P, Pair>(b2, pmm<P, Pair>(lhst, a9));
+}
+
+// The same on the bf16 instructions, for inputs of N parts.
+template <int N, bool Pair>
+__device__ __forceinline__ PTm<32, Pair> split_polynomial(const PTm<32, Pair>& a, const Ident<32>& id,
+                                                          const PartLds& at) {
+  PParts<Pair, N> ya;
+  const PLeft<Pair, N> xa = to_left<N, Pair>(a, ya, at);
+  const PTm<32, Pair> a2 = split_pmm<Pair>(xa, ya);
+  const PTm<32, Pair> a3 = split_pmm<Pair>(xa, psplit<3, Pair>(a2));
+  PParts<Pair> y3, unused;
+  const PLeft<Pair, 3> x3 = to_left<3, Pair>(a3, y3, at);
+  const PTm<32, Pair> a6 = split_pmm<Pair>(x3, y3);
+  const PLeft<Pair, 3> x1 = to_left<3, Pair>(combine<0, 32, Pair>(a, a2, a3, a6, id), unused, at);
+  const PParts<Pair> y5 = psplit<3, Pair>(combine<4, 32, Pair>(a, a2, a3, a6, id));
+  const PTm<32, Pair> b4 = combine<3, 32, Pair>(a, a2, a3, a6, id);
+  const PTm<32, Pair> b3 = combine<2, 32, Pair>(a, a2, a3, a6, id);
+  const PTm<32, Pair> b2 = combine<1, 32, Pair>(a, a2, a3, a6, id);
+  const PTm<32, Pair> a9 = padd<32, Pair>(split_pmm<Pair>(x1, y5), b4);
+  const PLeft<Pair, 3> x9 = to_left<3, Pair>(padd<32, Pair>(b3, a9), unused, at);
+  return padd<32, Pair>(b2, split_pmm<Pair>(x9, psplit<3, Pair>(a9)));
+}
+
 template <typename T, int P, bool Pair, int XL, int GL, bool Full>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P, Pair>(), 8))) void expm_tile_kernel(
     ExpmArgs args) {
   using C = TileCfg<P>;
   constexpr int R = C::R;
-  __shared__ float buf[2 * P * (P + 1)];
-  const int lane = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) char lds[kTileLds<P, Pair>];
+  float* const buf = reinterpret_cast<float*>(lds);
+  const int thread = threadIdx.x;
   const int n = Full ? P : args.n;
-  const TileSrc sx = make_src<T, P>(args.x, XL, n, lane);
-  const TileSrc sg = make_src<T, P>(args.g, GL, n, lane);
 
   int64_t b = blockIdx.x;
-  const int dreg_lane = C::diag_reg(lane);
   Ident<P> id_lane;
   if constexpr (P == 16) {
-    id_lane = make_ident<P>(dreg_lane);
+    id_lane = make_ident<P>(C::diag_reg(thread));
 #pragma unroll
     for (int r = 0; r < R; ++r) asm volatile("" : "+v"(id_lane.b3.v[r]), "+v"(id_lane.b4.v[r]));
   }
   for (; b < args.batch; b += gridDim.x) {
-    // For P = 32, opaque per matrix so that the identity terms are selected
-    // where they are used instead of being kept live across the loop.
+    // P = 32 derives everything that depends on the lane or the strides afresh
+    // for each matrix and for its store, so that offsets, bounds predicates and
+    // identity terms are not kept live across the products: registers these
+    // kernels do not have, on a grid where a wavefront seldom sees a second
+    // matrix.  P = 16 keeps them.
+    int lane = P == 32 ? fresh_lane() : thread;
+    int64_t major_x = XL == kLoadCols ? args.x.sc : args.x.sr, major_g = GL == kLoadCols ? args.g.sc : args.g.sr;
+    if constexpr (P == 32) asm volatile("" : "+s"(major_x), "+s"(major_g));
+    const TileSrc sx = make_src<T, P>(args.x, XL, major_x, n, lane);
+    const TileSrc sg = make_src<T, P>(args.g, GL, major_g, n, lane);
     Ident<P> id;
     if constexpr (P == 16) {
       id = id_lane;
     } else {
-      int dreg = dreg_lane;
-      asm volatile("" : "+v"(dreg));
-      id = make_ident<P>(dreg);
+      id = make_ident<P>(C::diag_reg(lane));
     }
-    // n < P = 32: the per-VGPR bounds predicates and offsets are formed
-    // afresh for each matrix from an opaque copy of the lane's offsets, so
-    // that they are not kept live across the loop (2R-3R registers these
-    // kernels do not have; P = 16 keeps them).
-    TileSrc sxm = sx, sgm = sg;
-    int lane_m = lane;
-    if constexpr (!Full && P == 32) {
-      asm volatile("" : "+v"(sxm.lane_off), "+v"(sgm.lane_off), "+v"(lane_m));
-    }
-    const Tm<P> lx = to_tile<T, P>(load_raw<T, P, Full>(sxm, b, n, lane_m));
+    const Tm<P> lx = to_tile<T, P>(load_raw<T, P, Full>(sx, b, n, lane));
     Tm<P> lg;
-    if constexpr (Pair) lg = to_tile<T, P>(load_raw<T, P, Full>(sgm, b, n, lane_m));
+    if constexpr (Pair) lg = to_tile<T, P>(load_raw<T, P, Full>(sg, b, n, lane));
 
-    // Both layouts of X (and G): the loaded one and its LDS transpose.
+    // The D layout of X and G and, for P = 16, of their transposes: the loaded
+    // one and its LDS transpose.
     PTm<P, Pair> a, at;
-    {
+    if constexpr (P == 16) {
       PTm<P, Pair> loaded;
       loaded.d = lx;
       if constexpr (Pair) loaded.u = lg;
@@ -473,6 +746,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
         a.u = GL == kLoadCols ? other.u : lg;
         at.u = GL == kLoadCols ? lg : other.u;
       }
+    } else {
+      a.d = XL == kLoadCols ? transpose<P>(lx, buf, lane) : lx;
+      if constexpr (Pair) a.u = GL == kLoadCols ? transpose<P>(lg, buf, lane) : lg;
     }
 
     int s;
@@ -481,10 +757,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
       Tm<P> nan;
 #pragma unroll
       for (int r = 0; r < R; ++r) nan.v[r] = __builtin_nanf("");
-      store_tile<T, P, Full>(args.out, b, n, lane_m, nan);
+      store_tile<T, P, Full>(args.out, b, n, lane, nan);
       if (lane == 0 && args.s_out) args.s_out[b] = -1;
       continue;
     }
+    s = __builtin_amdgcn_readfirstlane(s);
 
     // Scale by 2^-s (csrc/MatrixExpSmall.cuh:362-367), the views' lazy
     // negation folded into the same exact multiply.
@@ -494,38 +771,44 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       a.d.v[r] *= scale_x;
-      at.d.v[r] *= scale_x;
-      if constexpr (Pair) {
-        a.u.v[r] *= scale_g;
-        at.u.v[r] *= scale_g;
+      if constexpr (Pair) a.u.v[r] *= scale_g;
+      if constexpr (P == 16) {
+        at.d.v[r] *= scale_x;
+        if constexpr (Pair) at.u.v[r] *= scale_g;
       }
     }
 
-    // Degree-18 polynomial (csrc/MatrixExpSmall.cuh:83-106): A^2 = A.A,
-    // A^3 = A.A^2, A^6 = A^3.A^3, A9 = B1.B5 + B4, T = B2 + (B3 + A9).A9.
-    const PTm<P, Pair> a2 = pmm<P, Pair>(at, a);
-    const PTm<P, Pair> a3 = pmm<P, Pair>(at, a2);
-    const PTm<P, Pair> a6 = pmm<P, Pair>(ptranspose<P, Pair>(a3, buf, lane), a3);
-    // The sums B1.B5 + B4, B3 + A9 and B2 + (..).A9 are formed after their
-    // products, as in the reference: starting the MFMA accumulations from B4
-    // and B2 instead raised the FP32 error 1.4-fold on average (measured over
-    // config 5 against the FP64 result and the reference's own arithmetic).
-    const PTm<P, Pair> b1t = ptranspose<P, Pair>(combine<0, P, Pair>(a, a2, a3, a6, id), buf, lane);
-    const PTm<P, Pair> b5 = combine<4, P, Pair>(a, a2, a3, a6, id);
-    const PTm<P, Pair> b1b5 = pmm<P, Pair>(b1t, b5);
-    const PTm<P, Pair> a9 = padd<P, Pair>(b1b5, combine<3, P, Pair>(a, a2, a3, a6, id));
-    const PTm<P, Pair> lhst = ptranspose<P, Pair>(padd<P, Pair>(combine<2, P, Pair>(a, a2, a3, a6, id), a9), buf, lane);
-    const PTm<P, Pair> b2 = combine<1, P, Pair>(a, a2, a3, a6, id);
-    PTm<P, Pair> res = padd<P, Pair>(b2, pmm<P, Pair>(lhst, a9));
-    if constexpr (Pair) {
-      // The last squaring forms only the U block (the output).
-      for (int i = 1; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, lane), res);
-      if (s > 0) res = pmm<P, Pair, false>(ptranspose<P, Pair>(res, buf, lane), res);
+    // The last squaring of a pair forms only the U block (the output).
+    PTm<P, Pair> res;
+    if constexpr (P == 16) {
+      const auto same_lane = [lane] { return lane; };
+      res = polynomial<P, Pair>(a, at, id, buf, same_lane);
+      for (int i = Pair ? 1 : 0; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, lane), res);
+      if (Pair && s > 0) res = pmm<P, Pair, !Pair>(ptranspose<P, Pair>(res, buf, lane), res);
     } else {
-      for (int i = 0; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, lane), res);
+      int i = 0;
+      if (splittable<T, Pair>(a)) {
+        const PartLds part_lds(lds, lane);
+        res = split_polynomial<kInputParts<T>, Pair>(a, id, part_lds);
+        for (; i < s; ++i) {
+          if (i >= kUncheckedSquarings && !squares_in_range<Pair>(res)) break;
+          PParts<Pair> y;
+          const PLeft<Pair, 3> x = to_left<3, Pair>(res, y, part_lds);
+          if (Pair && i == s - 1) {
+            res = split_pmm<Pair, !Pair>(x, y);
+          } else {
+            res = split_pmm<Pair>(x, y);
+          }
+        }
+      } else {
+        res = polynomial<P, Pair>(a, ptranspose<P, Pair>(a, buf, fresh_lane()),
+                                  make_ident<P>(C::diag_reg(fresh_lane())), buf, fresh_lane);
+      }
+      for (; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
+      lane = fresh_lane();
     }
 
-    store_tile<T, P, Full>(args.out, b, n, lane_m, Pair ? res.u : res.d);
+    store_tile<T, P, Full>(args.out, b, n, lane, Pair ? res.u : res.d);
     if (lane == 0 && args.s_out) args.s_out[b] = s;
   }
 }
