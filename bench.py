@@ -35,7 +35,7 @@ Reported (in full in the report, summarised in the line):
 * ``configs`` -- configs 3-5 (BF16 N=4 sweep, strided FP32 N=16, FP16 N=32 and
   the same shape in FP32) plus ``p8`` / ``c2s8`` with their own rooflines (HBM
   bytes at 8 TB/s, product flops from each matrix's own squaring count at the
-  FP32 matrix peak), and ``hc`` -- the fused stream mixing ``fh.mix_streams``
+  FP32 matrix peak, for n >= 17 at a sixth of the bf16 matrix peak), and ``hc`` -- the fused stream mixing ``fh.mix_streams``
   (y = exp(h) x, 16,384 tokens x 4 streams x 4,096 columns, BF16) forward and
   forward + backward, each fused kernel against the HBM roofline, beside the
   composed ``fh.matrix_exp(h) @ x`` on the same inputs;
@@ -69,6 +69,7 @@ for _p in (str(ROOT / "flash-hyperconnections_amd"), str(ROOT)):
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 MFMA_F32_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix
+MFMA_SPLIT_PEAK_TFLOPS = 2500.0 / 6  # FP32 products as six bf16 ones (n >= 17), dense bf16 matrix
 VALU_F32_UNPACKED_TFLOPS = 78.6  # 256 CUs x 4 SIMDs x 16 lanes x 2 flops x 2.4 GHz (packed FP32 is not used)
 METRIC = "matrices/sec fwd+bwd (N=4 B=2^20, N=32 B=32768); % HBM/MFMA roofline"
 
@@ -239,7 +240,7 @@ def measure_config(name: str, torch, fh, steps: int, warmup: int, trials: int, d
     bytes_bwd = b * n * n * 3 * e
     flops_fwd = float(((5 + s_f) * 2 * n**3).sum())
     flops_bwd = float(((5 + s_b) * 3 * 2 * n**3).sum())
-    peak = MFMA_F32_PEAK_TFLOPS
+    peak = MFMA_F32_PEAK_TFLOPS if n <= 16 else MFMA_SPLIT_PEAK_TFLOPS
     bound, t_ideal = roofline_times(bytes_fwd + bytes_bwd, flops_fwd + flops_bwd, peak)
     bound_fwd, t_f = roofline_times(bytes_fwd, flops_fwd, peak)
     bound_bwd, t_b = roofline_times(bytes_bwd, flops_bwd, peak)
