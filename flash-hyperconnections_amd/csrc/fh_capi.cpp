@@ -7,6 +7,7 @@
 #include <string>
 
 #include "fh_kernels.h"
+#include "fh_rows.h"
 #include "flash_hypercons.h"
 
 namespace {
@@ -128,6 +129,13 @@ constexpr int64_t kSpan = int64_t{1} << 31;  // bytes one token's rows may span 
 bool stream_rows_ok(const void* p, const int64_t* st, int64_t cols, int dtype) {
   const int64_t v = 16 / element_size(dtype);
   return st != nullptr && aligned(p, 16) && st[2] == 1 && st[0] >= 0 && st[1] >= 0 && st[0] % v == 0 &&
+         st[1] % v == 0 && cols % v == 0;
+}
+
+// The same with dwords for vectors: what the fused kernels' ragged variants read.
+bool dword_rows_ok(const void* p, const int64_t* st, int64_t cols, int dtype) {
+  const int64_t v = 4 / element_size(dtype);
+  return st != nullptr && aligned(p, 4) && st[2] == 1 && st[0] >= 0 && st[1] >= 0 && st[0] % v == 0 &&
          st[1] % v == 0 && cols % v == 0;
 }
 
@@ -275,6 +283,33 @@ int fh_hc_mix_backward(const void* h, const int64_t h_strides[3], int h_neg, con
   if (batch == 0) return FH_OK;
   const hipError_t err = fh::launch_hc_mix(fh::hc_operand(h, h_strides, h_neg, dtype), x, x_strides, grad,
                                            grad_strides, dx, dh, de_out, dtype, batch, n, cols, stream);
+  if (err != hipSuccess) return fail(FH_ERR_LAUNCH, std::string("kernel launch failed: ") + hipGetErrorString(err));
+  g_error.clear();
+  return FH_OK;
+}
+
+int fh_hc_mix_dwords(const void* h, const int64_t h_strides[3], int h_neg, const void* x, const int64_t x_strides[3],
+                     const void* grad, const int64_t* grad_strides, void* dh, void* out, float* aux, int dtype,
+                     int64_t batch, int n, int64_t cols, hipStream_t stream) {
+  if (n < 2 || n > 4 || !known_dtype(dtype) || batch < 0 || cols < 1)
+    return fail(FH_ERR_INVALID_ARGUMENT,
+                "hc_mix: expected H [B, n, n] and X [B, n, C] with 2 <= n <= 4, C >= 1, in float32, float16, or "
+                "bfloat16");
+  if (batch == 0) return FH_OK;
+  if (h == nullptr || h_strides == nullptr || x == nullptr || x_strides == nullptr || out == nullptr ||
+      (grad != nullptr && (grad_strides == nullptr || dh == nullptr)))
+    return fail(FH_ERR_INVALID_ARGUMENT, "hc_mix: null pointer");
+  if (!dword_rows_ok(x, x_strides, cols, dtype) || (grad != nullptr && !dword_rows_ok(grad, grad_strides, cols, dtype)) ||
+      !aligned(out, 4))
+    return fail(FH_ERR_INVALID_ARGUMENT, "hc_mix: X and dY need contiguous, 4-byte aligned rows of whole dwords");
+  // The span of the rows padded to whole vectors: the limit of the padded layout.
+  const int64_t v = 16 / element_size(dtype);
+  const int64_t padded = cols < kSpan ? (cols + v - 1) / v * v : cols;
+  if (!stream_span_ok(x_strides, n, padded, dtype) ||
+      (grad != nullptr && !stream_span_ok(grad_strides, n, padded, dtype)))
+    return fail(FH_ERR_INVALID_ARGUMENT, span_message("hc_mix"));
+  const hipError_t err = fh::launch_hc_mix(fh::hc_operand(h, h_strides, h_neg, dtype), x, x_strides, grad,
+                                           grad_strides, out, dh, aux, dtype, batch, n, cols, stream);
   if (err != hipSuccess) return fail(FH_ERR_LAUNCH, std::string("kernel launch failed: ") + hipGetErrorString(err));
   g_error.clear();
   return FH_OK;

@@ -19,12 +19,13 @@ hipError_t launch_p4(const ExpmArgs& args, int dtype, bool pair, hipStream_t str
 // (launch_oct16), the Frechet derivative with 4.
 hipError_t launch_oct(const ExpmArgs& args, int dtype, bool pair, hipStream_t stream);
 hipError_t launch_oct16(const ExpmArgs& args, int dtype, hipStream_t stream);
-// P in {16, 32}: one wavefront per matrix on 16x16x4 / 32x32x2 MFMA.
+// P in {16, 32}: one wavefront per matrix on 16x16x4 FP32 / 32x32x16 bf16 MFMA.
 hipError_t launch_tile(const ExpmArgs& args, int dtype, int P, bool pair, hipStream_t stream);
 // Fused hyper-connection stream mixing (n = 2..4): gy == nullptr selects the
 // forward Y = exp(H) X into `out`; otherwise the backward dX = exp(H)^T dY into
 // `out` and dH = L(H^T, dY X^T) into `dh`.  `xs` / `gs`: element strides
-// (token, row) of X / dY, whose columns are contiguous.  `aux` (may be null):
+// (token, row) of X / dY, whose columns are contiguous; bases, strides and C
+// are whole 16-byte vectors, or whole dwords (another kernel).  `aux` (may be null):
 // FP32 [B, n, n] copy of exp(H) (forward) or dY X^T (backward).
 // H of the stream mixing as an element-class operand.
 Operand hc_operand(const void* h, const int64_t strides[3], int neg, int dtype);

@@ -126,6 +126,41 @@ __device__ __forceinline__ void store16(U32x4 w, __amdgpu_buffer_rsrc_t rs, int3
   __builtin_amdgcn_raw_buffer_store_b128(w, rs, voff, 0, kStreamPolicy);
 }
 
+// One lane's vector of a row of which `left` elements remain.  Ragged: rows in
+// whole dwords at any dword (a multi-dword buffer access needs no more), the
+// row's last vector by dwords, zero past its end.  The lanes hold the columns
+// they hold of a row padded to whole vectors, so the results are the same bits.
+// Against padding the operands and unpadding the result (ten launches a step),
+// us forward and forward + backward: 4096 x 4 x 1026 BF16 69.8 -> 20.5 and
+// 213 -> 57 (host), 4096 x 4 x 4093 FP32 361 -> 117 and 964 -> 299 (4.6 and
+// 4.5 TB/s), 16384 x 3 x 1538 FP16 195 -> 64 and 506 -> 171.
+template <typename T, bool Ragged>
+__device__ __forceinline__ U32x4 load_vec(__amdgpu_buffer_rsrc_t rs, int32_t voff, int left) {
+  constexpr int V = Vec<T>::V;
+  if constexpr (!Ragged) return left > 0 ? load16(rs, voff) : U32x4{0, 0, 0, 0};
+  U32x4 w{0, 0, 0, 0};
+  if (left >= V) {
+    w = load16(rs, voff);
+  } else {
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (d * (V / 4) < left) w[d] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff + 4 * d, 0, kStreamPolicy);
+  }
+  return w;
+}
+
+template <typename T, bool Ragged>
+__device__ __forceinline__ void store_vec(U32x4 w, __amdgpu_buffer_rsrc_t rs, int32_t voff, int left) {
+  constexpr int V = Vec<T>::V;
+  if (Ragged ? left >= V : left > 0) {
+    store16(w, rs, voff);
+  } else if constexpr (Ragged) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (d * (V / 4) < left) __builtin_amdgcn_raw_buffer_store_b32(w[d], rs, voff + 4 * d, 0, kStreamPolicy);
+  }
+}
+
 // Wavefronts of a workgroup that share one token's columns, for passes of
 // `width` columns: four, or fewer when C has fewer passes, in which case the
 // others take other tokens.  By C alone (see above).
@@ -220,7 +255,7 @@ constexpr int kChunks = 4;
 constexpr int kChunksBwd = 2;
 
 // Forward: Y_b = E_b X_b, row i of Y = sum_k E[i][k] X[k] (fmaf chain k = 0..n-1 from +0).
-template <typename T, int N>
+template <typename T, int N, bool Ragged>
 __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
   __shared__ __attribute__((aligned(16))) float etile_mem[kWaves][kTokens * 16];
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
@@ -241,7 +276,7 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
       const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
       for (int k = 0; k < N; ++k)
-        raw[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
+        raw[u][k] = load_vec<T, Ragged>(xs, (k * xr_step + c) * es, cols - c);
     }
   };
   exp_tokens<T, N>(a, sh, lane, wave, etile);
@@ -266,7 +301,7 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
             for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
             y.f[v] = acc;
           }
-          if (c < cols) store16(pack<T>(y), ys, (i2 * cols + c) * es);
+          store_vec<T, Ragged>(pack<T>(y), ys, (i2 * cols + c) * es, cols - c);
         }
       }
     }
@@ -335,7 +370,7 @@ __device__ __forceinline__ float wave_sum(const float (&v)[M], int lane) {
 // Backward: dX row k = sum_r E[r][k] dY[r] (fmaf chain r = 0..n-1 from +0);
 // dE[r][k] = sum_c dY[r][c] X[k][c] (per lane in column order, then
 // wave_sum, then the wavefronts' parts in order); dH = L(H^T, dE).
-template <typename T, int N>
+template <typename T, int N, bool Ragged>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_mix_bwd_kernel(HcArgs a) {
   __shared__ __attribute__((aligned(16))) float etile_mem[kWaves][kTokens * 16];
   __shared__ __attribute__((aligned(16))) float gtile_mem[kWaves][kTokens * 16];  // dE by column part
@@ -367,8 +402,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
         const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          xr[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
-          gr[u][k] = c < cols ? load16(gs, (k * gr_step + c) * es) : U32x4{0, 0, 0, 0};
+          xr[u][k] = load_vec<T, Ragged>(xs, (k * xr_step + c) * es, cols - c);
+          gr[u][k] = load_vec<T, Ragged>(gs, (k * gr_step + c) * es, cols - c);
         }
       }
 #pragma unroll
@@ -390,7 +425,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
             for (int r = 1; r < N; ++r) d = __builtin_fmaf(e.v[4 * r + k], gv[r].f[v], d);
             dx.f[v] = d;
           }
-          if (c < cols) store16(pack<T>(dx), ds, (k * cols + c) * es);
+          store_vec<T, Ragged>(pack<T>(dx), ds, (k * cols + c) * es, cols - c);
         }
 #pragma unroll
         for (int r = 0; r < N; ++r)
@@ -712,8 +747,17 @@ hipError_t launch_sets(void (*kernel)(Args), Args a, int most, hipStream_t strea
 // has a Frechet polynomial a set as well, 195 / 178 / 183 and 87 / 81 / 79.
 template <typename T, int N, bool Backward>
 hipError_t launch_one(HcArgs a, hipStream_t stream) {
-  const auto kernel = Backward ? hc_mix_bwd_kernel<T, N> : hc_mix_fwd_kernel<T, N>;
-  a.parts = column_parts(a.cols, 64 * Vec<T>::V * kChunksBwd);
+  // Whole 16-byte vectors everywhere, or rows in whole dwords at any dword.  The
+  // line lies at the dword because buffer accesses of a dword or more need that
+  // alignment: rows of an odd number of 16-bit values are padded by the caller.
+  constexpr int V = Vec<T>::V;
+  const bool ragged = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.gy) |
+                        reinterpret_cast<uintptr_t>(a.out)) % 16 != 0) ||
+                      ((a.cols | a.xb | a.xr | a.gb | a.gr) % V != 0);
+  const auto kernel = Backward ? (ragged ? hc_mix_bwd_kernel<T, N, true> : hc_mix_bwd_kernel<T, N, false>)
+                               : (ragged ? hc_mix_fwd_kernel<T, N, true> : hc_mix_fwd_kernel<T, N, false>);
+  // A ragged row shares its columns as the row padded to whole vectors would.
+  a.parts = column_parts((a.cols + V - 1) / V * V, 64 * V * kChunksBwd);
   return launch_sets(kernel, a, Backward ? kTokens : kTokens / 2, stream);
 }
 

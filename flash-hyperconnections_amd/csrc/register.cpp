@@ -31,6 +31,7 @@
 #include <optional>
 #include <tuple>
 
+#include "fh_rows.h"
 #include "flash_hypercons.h"
 
 namespace flash_hypercons {
@@ -163,6 +164,32 @@ at::Tensor streamable(const at::Tensor& x) {
   return p;
 }
 
+// Rows that hold no whole number of vectors but whole dwords (n <= 4): read in
+// place by the kernels' ragged variants, or after one plain copy.
+struct DwordRows {
+  at::Tensor t;
+  int64_t strides[3];
+  explicit DwordRows(const at::Tensor& x) : t(x) {
+    if (!fits()) t = x.resolve_neg().contiguous();
+    if (!fits()) t = t.clone(at::MemoryFormat::Contiguous);
+  }
+
+ private:
+  // The strides of dimensions of one entry are free: a tensor that counts as
+  // contiguous may hold anything there.
+  bool fits() {
+    constexpr int64_t kSpan = int64_t{1} << 31;
+    const int64_t es = static_cast<int64_t>(t.element_size()), v = 4 / es;
+    const int64_t padded = (t.size(2) + 16 / es - 1) / (16 / es) * (16 / es);
+    strides[0] = t.size(0) == 1 ? 0 : t.stride(0);
+    strides[1] = t.stride(1);
+    strides[2] = t.size(2) == 1 ? 1 : t.stride(2);
+    return !t.is_neg() && strides[2] == 1 && strides[0] >= 0 && strides[1] >= 0 && strides[0] % v == 0 &&
+           strides[1] % v == 0 && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 4 == 0 && strides[1] < kSpan &&
+           ((t.size(1) - 1) * strides[1] + padded) * es < kSpan;
+  }
+};
+
 std::tuple<at::Tensor, at::Tensor, at::Tensor> mix_run(const at::Tensor& h, const at::Tensor& x,
                                                        const std::optional<at::Tensor>& grad, bool want_aux) {
   check_mix(h, x);
@@ -171,6 +198,23 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> mix_run(const at::Tensor& h, cons
                         "mix_streams: grad must match x");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(h.device());
   const int64_t B = h.size(0), n = h.size(1), C = x.size(2);
+  const int64_t es = static_cast<int64_t>(x.element_size());
+  if (B > 0 && C * es % 16 != 0 && C * es % 4 == 0) {
+    // Padding the rows and unpadding the results instead (zero fills and copies,
+    // below) made ten launches of a step that has two kernels.
+    const DwordRows xr(x);
+    at::Tensor out = at::empty({B, n, C}, x.options());
+    at::Tensor dh = grad ? at::empty({B, n, n}, h.options()) : at::Tensor();
+    at::Tensor aux = want_aux ? at::empty({B, n, n}, h.options().dtype(at::kFloat)) : at::Tensor();
+    const std::optional<DwordRows> gr = grad ? std::make_optional<DwordRows>(*grad) : std::nullopt;
+    const View hv = view_of(h);
+    check_status(fh_hc_mix_dwords(hv.data, hv.strides, hv.neg, xr.t.const_data_ptr(), xr.strides,
+                                  gr ? gr->t.const_data_ptr() : nullptr, gr ? gr->strides : nullptr,
+                                  grad ? dh.mutable_data_ptr() : nullptr, out.mutable_data_ptr(),
+                                  want_aux ? aux.mutable_data_ptr<float>() : nullptr, dtype_code(h.scalar_type()), B,
+                                  static_cast<int>(n), C, current_stream()));
+    return {out, dh, aux};
+  }
   const at::Tensor xs = streamable(x);
   const int64_t Cp = xs.size(2);
   at::Tensor out = at::empty({B, n, Cp}, x.options());
