@@ -1,8 +1,8 @@
 // P in {16, 32} kernel (n = 9..32): one 64-lane wavefront per matrix, every
 // product on the matrix cores: P = 16 on v_mfma_f32_16x16x4_f32, P = 32 on
 // v_mfma_f32_32x32x16_bf16 with each FP32 value as the sum of three bf16 ones
-// (and on v_mfma_f32_32x32x2_f32 where that sum would not hold; the section on
-// bf16 below).
+// (and late squarings of very large operands on v_mfma_f32_32x32x2_f32; the
+// section on bf16 below).
 //
 // Layout: a P x P matrix occupies R = P*P/64 VGPRs per lane in the MFMA
 // accumulator ("D") layout: lane l, VGPR r holds M[row(l, r)][l % P] with
@@ -367,26 +367,34 @@ __device__ __forceinline__ PTm<32, Pair> split_pmm(const PLeft<Pair, NX>& x, con
   return out;
 }
 
-// bf16 MFMAs read subnormal operands as zero.  The parts of v keep its bits while
-// |v| is 0 or at least 2^-100; matrices with smaller entries (scaled by 2^-s)
-// take the FP32 instructions.  FP16 inputs cannot have any: s <= 22.
-template <typename T, bool Pair>
-__device__ __forceinline__ bool splittable(const PTm<32, Pair>& a) {
-  if constexpr (T::code == F16::code) return true;
-  constexpr uint32_t kLeast = ((127u - 100u) << 24) - 1u;
-  // Twice the magnitude's bits minus one: zero becomes the largest value.
-  uint32_t least = ~0u;
+// bf16 MFMAs read subnormal operands as zero, and the low part of a value below
+// 2^-103 may be one.  So every operand of a product is 2^24 times its matrix or
+// more: its parts are multiples of 2^24 * 2^-149, all normal, and the products
+// and sums of values that FP32 holds at all are normal as well.  The scales are
+// powers of two: they go into the factor 2^-s of the input and into the
+// polynomial's coefficients and cost a multiply per entry only of A^3 and of a
+// result.  kScale[k] are the exponents of I, A, A^2, A^3 and A^6, kOperandScale
+// those of the operands B1, B5 and exp.
+constexpr int kOperandScale = 24;
+constexpr int kScale[5] = {0, kOperandScale, 2 * kOperandScale, 32, 64};
+
+__device__ constexpr float pow2(int e) { return e < 0 ? 0.5f * pow2(e + 1) : e > 0 ? 2.f * pow2(e - 1) : 1.f; }
+
+// m * 2^e, of a pair U alone when nothing reads D.
+template <bool Pair, bool WantD = true>
+__device__ __forceinline__ void rescale(PTm<32, Pair>& m, int e) {
+  float factor = __builtin_ldexpf(1.f, e);
+  asm("" : "+v"(factor));  // a VGPR: an SGPR operand costs a full-rate instruction 1.5x
 #pragma unroll
   for (int r = 0; r < TileCfg<32>::R; ++r) {
-    least = min(least, (__float_as_uint(a.d.v[r]) << 1) - 1u);
-    if constexpr (Pair) least = min(least, (__float_as_uint(a.u.v[r]) << 1) - 1u);
+    if constexpr (WantD) m.d.v[r] *= factor;
+    if constexpr (Pair) m.u.v[r] *= factor;
   }
-  return __builtin_amdgcn_ballot_w64(least < kLeast) == 0;
 }
 
-// Whether squaring `m` keeps every partial product and sum finite (64 terms
-// below 2^120); otherwise a low part's product could overflow to the opposite
-// infinity and make NaN of a result that is infinite.
+// Whether squaring the scaled `m` keeps every partial product and sum finite (64
+// terms below 2^120); otherwise a low part's product could overflow to the
+// opposite infinity and make NaN of a result that is infinite.
 template <bool Pair>
 __device__ __forceinline__ bool squares_in_range(const PTm<32, Pair>& m) {
   float top = 0.f;
@@ -399,48 +407,45 @@ __device__ __forceinline__ bool squares_in_range(const PTm<32, Pair>& m) {
 }
 
 // The polynomial has norm at most exp(theta18) = e^3.01 and i squarings raise
-// that to exp(theta18 2^i): four rounds (operands to e^24, results to e^48) need
-// no check.
+// that to exp(theta18 2^i): four rounds (operands to e^24, results to e^48, 2^118
+// with the scale of both sides) need no check.
 constexpr int kUncheckedSquarings = 4;
 
 // c0*I in the D layout for the two combines with an identity term (B3 and B4,
 // reference csrc/MatrixExpSmall.cuh:268-281), from `dreg`, the VGPR of this
-// lane's diagonal entry (-1 for none).  P = 16 keeps the 2R values in
+// lane's diagonal entry (-1 for none).  P = 16 keeps these 2R values in
 // registers for the whole kernel (it has registers to spare); P = 32 selects
 // them where they are used.
-template <int P>
-struct Ident {
-  int dreg;
-  __device__ __forceinline__ float value(int k, int r) const { return dreg == r ? kCoef[k][0] : 0.f; }
-};
-template <>
-struct Ident<16> {
+struct Ident16 {
   Tm<16> b3, b4;
+  __device__ __forceinline__ explicit Ident16(int dreg) {
+#pragma unroll
+    for (int r = 0; r < TileCfg<16>::R; ++r) {
+      b3.v[r] = dreg == r ? kCoef[2][0] : 0.f;
+      b4.v[r] = dreg == r ? kCoef[3][0] : 0.f;
+    }
+  }
   __device__ __forceinline__ float value(int k, int r) const { return k == 2 ? b3.v[r] : b4.v[r]; }
 };
-template <int P>
-__device__ __forceinline__ Ident<P> make_ident(int dreg) {
-  Ident<P> id;
-  if constexpr (P == 16) {
-#pragma unroll
-    for (int r = 0; r < TileCfg<P>::R; ++r) {
-      id.b3.v[r] = dreg == r ? kCoef[2][0] : 0.f;
-      id.b4.v[r] = dreg == r ? kCoef[3][0] : 0.f;
-    }
-  } else {
-    id.dreg = dreg;
-  }
-  return id;
-}
+// The same scaled by 2^Out.
+template <int Out>
+struct Ident32 {
+  static constexpr float kB3 = kCoef[2][0] * pow2(Out), kB4 = kCoef[3][0] * pow2(Out);
+  int dreg;
+  __device__ __forceinline__ float value(int k, int r) const { return dreg == r ? (k == 2 ? kB3 : kB4) : 0.f; }
+};
 
 // B(K+1) = c0*I + c1*A + c2*A^2 + c3*A^3 + c6*A^6 (reference
 // csrc/MatrixExpSmall.cuh:268-281), the contracted chain with zero
-// coefficients skipped; the identity term (D only) comes from `id`.
-template <int K, int P, bool Pair>
+// coefficients skipped; the identity term (D only) comes from `id`.  At P = 32
+// the powers are scaled by 2^kScale and B by 2^Out.
+template <int K, int Out = 0, int P, bool Pair, typename Id>
 __device__ __forceinline__ PTm<P, Pair> combine(const PTm<P, Pair>& a, const PTm<P, Pair>& a2,
-                                                const PTm<P, Pair>& a3, const PTm<P, Pair>& a6, const Ident<P>& id) {
+                                                const PTm<P, Pair>& a3, const PTm<P, Pair>& a6, const Id& id) {
   using C = TileCfg<P>;
-  constexpr float c0 = kCoef[K][0], c1 = kCoef[K][1], c2 = kCoef[K][2], c3 = kCoef[K][3], c6 = kCoef[K][4];
+  const auto scale = [](int k) constexpr { return P == 32 ? pow2(Out - kScale[k]) : 1.f; };
+  constexpr float c0 = kCoef[K][0], c1 = kCoef[K][1] * scale(1), c2 = kCoef[K][2] * scale(2),
+                  c3 = kCoef[K][3] * scale(3), c6 = kCoef[K][4] * scale(4);
   static_assert(c0 == 0.f || K == 2 || K == 3, "identity terms are B3 and B4");
   PTm<P, Pair> b;
 #pragma unroll
@@ -656,39 +661,41 @@ static_assert(3 * kPartBytes >= 4 * 32 * 33);
 // 32768 32 x 32 matrices against the FP64 result and the reference's own
 // arithmetic).
 //
-// On the FP32 instructions; `at` is a's transpose and `lane()` the lane.
-template <int P, bool Pair, typename Lane>
-__device__ __forceinline__ PTm<P, Pair> polynomial(const PTm<P, Pair>& a, const PTm<P, Pair>& at, const Ident<P>& id,
-                                                   float* buf, Lane lane) {
-  const PTm<P, Pair> a2 = pmm<P, Pair>(at, a);
-  const PTm<P, Pair> a3 = pmm<P, Pair>(at, a2);
-  const PTm<P, Pair> a6 = pmm<P, Pair>(ptranspose<P, Pair>(a3, buf, lane()), a3);
-  const PTm<P, Pair> b1t = ptranspose<P, Pair>(combine<0, P, Pair>(a, a2, a3, a6, id), buf, lane());
-  const PTm<P, Pair> b5 = combine<4, P, Pair>(a, a2, a3, a6, id);
-  const PTm<P, Pair> b1b5 = pmm<P, Pair>(b1t, b5);
-  const PTm<P, Pair> a9 = padd<P, Pair>(b1b5, combine<3, P, Pair>(a, a2, a3, a6, id));
-  const PTm<P, Pair> lhst =
-      ptranspose<P, Pair>(padd<P, Pair>(combine<2, P, Pair>(a, a2, a3, a6, id), a9), buf, lane());
-  const PTm<P, Pair> b2 = combine<1, P, Pair>(a, a2, a3, a6, id);
-  return padd<P, Pair>(b2, pmm<P, Pair>(lhst, a9));
+// P = 16, on the FP32 instructions; `at` is a's transpose.
+template <bool Pair>
+__device__ __forceinline__ PTm<16, Pair> polynomial(const PTm<16, Pair>& a, const PTm<16, Pair>& at, const Ident16& id,
+                                                    float* buf, int lane) {
+  const PTm<16, Pair> a2 = pmm<16, Pair>(at, a);
+  const PTm<16, Pair> a3 = pmm<16, Pair>(at, a2);
+  const PTm<16, Pair> a6 = pmm<16, Pair>(ptranspose<16, Pair>(a3, buf, lane), a3);
+  const PTm<16, Pair> b1t = ptranspose<16, Pair>(combine<0>(a, a2, a3, a6, id), buf, lane);
+  const PTm<16, Pair> b5 = combine<4>(a, a2, a3, a6, id);
+  const PTm<16, Pair> b1b5 = pmm<16, Pair>(b1t, b5);
+  const PTm<16, Pair> a9 = padd<16, Pair>(b1b5, combine<3>(a, a2, a3, a6, id));
+  const PTm<16, Pair> lhst = ptranspose<16, Pair>(padd<16, Pair>(combine<2>(a, a2, a3, a6, id), a9), buf, lane);
+  const PTm<16, Pair> b2 = combine<1>(a, a2, a3, a6, id);
+  return padd<16, Pair>(b2, pmm<16, Pair>(lhst, a9));
 }
 
-// The same on the bf16 instructions, for inputs of N parts.
+// P = 32, on the bf16 instructions, for inputs of N parts: from 2^24 A to 2^96 T.
+constexpr int kPolynomialScale = 4 * kOperandScale;
 template <int N, bool Pair>
-__device__ __forceinline__ PTm<32, Pair> split_polynomial(const PTm<32, Pair>& a, const Ident<32>& id,
-                                                          const PartLds& at) {
+__device__ __forceinline__ PTm<32, Pair> split_polynomial(const PTm<32, Pair>& a, int dreg, const PartLds& at) {
+  constexpr int kB = kOperandScale;  // B1 and B5; twice that B1.B5, B3 and B4
+  const Ident32<2 * kB> id{dreg};
   PParts<Pair, N> ya;
   const PLeft<Pair, N> xa = to_left<N, Pair>(a, ya, at);
   const PTm<32, Pair> a2 = split_pmm<Pair>(xa, ya);
-  const PTm<32, Pair> a3 = split_pmm<Pair>(xa, psplit<3, Pair>(a2));
+  PTm<32, Pair> a3 = split_pmm<Pair>(xa, psplit<3, Pair>(a2));
+  rescale<Pair>(a3, kScale[3] - kScale[1] - kScale[2]);
   PParts<Pair> y3, unused;
   const PLeft<Pair, 3> x3 = to_left<3, Pair>(a3, y3, at);
   const PTm<32, Pair> a6 = split_pmm<Pair>(x3, y3);
-  const PLeft<Pair, 3> x1 = to_left<3, Pair>(combine<0, 32, Pair>(a, a2, a3, a6, id), unused, at);
-  const PParts<Pair> y5 = psplit<3, Pair>(combine<4, 32, Pair>(a, a2, a3, a6, id));
-  const PTm<32, Pair> b4 = combine<3, 32, Pair>(a, a2, a3, a6, id);
-  const PTm<32, Pair> b3 = combine<2, 32, Pair>(a, a2, a3, a6, id);
-  const PTm<32, Pair> b2 = combine<1, 32, Pair>(a, a2, a3, a6, id);
+  const PLeft<Pair, 3> x1 = to_left<3, Pair>(combine<0, kB>(a, a2, a3, a6, id), unused, at);
+  const PParts<Pair> y5 = psplit<3, Pair>(combine<4, kB>(a, a2, a3, a6, id));
+  const PTm<32, Pair> b4 = combine<3, 2 * kB>(a, a2, a3, a6, id);
+  const PTm<32, Pair> b3 = combine<2, 2 * kB>(a, a2, a3, a6, id);
+  const PTm<32, Pair> b2 = combine<1, kPolynomialScale>(a, a2, a3, a6, id);
   const PTm<32, Pair> a9 = padd<32, Pair>(split_pmm<Pair>(x1, y5), b4);
   const PLeft<Pair, 3> x9 = to_left<3, Pair>(padd<32, Pair>(b3, a9), unused, at);
   return padd<32, Pair>(b2, split_pmm<Pair>(x9, psplit<3, Pair>(a9)));
@@ -705,11 +712,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
   const int n = Full ? P : args.n;
 
   int64_t b = blockIdx.x;
-  Ident<P> id_lane;
+  Ident16 id(P == 16 ? C::diag_reg(thread) : -1);
   if constexpr (P == 16) {
-    id_lane = make_ident<P>(C::diag_reg(thread));
 #pragma unroll
-    for (int r = 0; r < R; ++r) asm volatile("" : "+v"(id_lane.b3.v[r]), "+v"(id_lane.b4.v[r]));
+    for (int r = 0; r < R; ++r) asm volatile("" : "+v"(id.b3.v[r]), "+v"(id.b4.v[r]));
   }
   for (; b < args.batch; b += gridDim.x) {
     // P = 32 derives everything that depends on the lane or the strides afresh
@@ -722,12 +728,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
     if constexpr (P == 32) asm volatile("" : "+s"(major_x), "+s"(major_g));
     const TileSrc sx = make_src<T, P>(args.x, XL, major_x, n, lane);
     const TileSrc sg = make_src<T, P>(args.g, GL, major_g, n, lane);
-    Ident<P> id;
-    if constexpr (P == 16) {
-      id = id_lane;
-    } else {
-      id = make_ident<P>(C::diag_reg(lane));
-    }
     const Tm<P> lx = to_tile<T, P>(load_raw<T, P, Full>(sx, b, n, lane));
     Tm<P> lg;
     if constexpr (Pair) lg = to_tile<T, P>(load_raw<T, P, Full>(sg, b, n, lane));
@@ -764,8 +764,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
     s = __builtin_amdgcn_readfirstlane(s);
 
     // Scale by 2^-s (csrc/MatrixExpSmall.cuh:362-367), the views' lazy
-    // negation folded into the same exact multiply.
-    const float scale = __builtin_ldexpf(1.f, -s);
+    // negation and the scale of P = 32's operands folded into the same exact
+    // multiply.
+    const float scale = __builtin_ldexpf(1.f, (P == 32 ? kOperandScale : 0) - s);
     const float scale_x = scale * args.x.sign;
     const float scale_g = scale * args.g.sign;
 #pragma unroll
@@ -781,30 +782,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
     // The last squaring of a pair forms only the U block (the output).
     PTm<P, Pair> res;
     if constexpr (P == 16) {
-      const auto same_lane = [lane] { return lane; };
-      res = polynomial<P, Pair>(a, at, id, buf, same_lane);
+      res = polynomial<Pair>(a, at, id, buf, lane);
       for (int i = Pair ? 1 : 0; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, lane), res);
       if (Pair && s > 0) res = pmm<P, Pair, !Pair>(ptranspose<P, Pair>(res, buf, lane), res);
     } else {
+      const PartLds part_lds(lds, lane);
+      res = split_polynomial<kInputParts<T>>(a, C::diag_reg(lane), part_lds);
+      int scale = s > 0 ? kOperandScale : 0;  // of res, as a power of two
+      rescale<Pair>(res, scale - kPolynomialScale);
       int i = 0;
-      if (splittable<T, Pair>(a)) {
-        const PartLds part_lds(lds, lane);
-        res = split_polynomial<kInputParts<T>, Pair>(a, id, part_lds);
-        for (; i < s; ++i) {
-          if (i >= kUncheckedSquarings && !squares_in_range<Pair>(res)) break;
-          PParts<Pair> y;
-          const PLeft<Pair, 3> x = to_left<3, Pair>(res, y, part_lds);
-          if (Pair && i == s - 1) {
-            res = split_pmm<Pair, !Pair>(x, y);
+      for (; i < s; ++i) {
+        if (i >= kUncheckedSquarings && !squares_in_range<Pair>(res)) break;
+        PParts<Pair> y;
+        const PLeft<Pair, 3> x = to_left<3, Pair>(res, y, part_lds);
+        const int twice = 2 * scale;
+        scale = i == s - 1 ? 0 : kOperandScale;
+        if (Pair && i == s - 1) {
+          res = split_pmm<Pair, !Pair>(x, y);
+          rescale<Pair, !Pair>(res, -twice);
+        } else {
+          res = split_pmm<Pair>(x, y);
+          // Two squarings of the polynomial, to e^12, fit without a rescaling between them.
+          if (i == 0 && s > 1) {
+            scale = twice;
           } else {
-            res = split_pmm<Pair>(x, y);
+            rescale<Pair>(res, scale - twice);
           }
         }
-      } else {
-        res = polynomial<P, Pair>(a, ptranspose<P, Pair>(a, buf, fresh_lane()),
-                                  make_ident<P>(C::diag_reg(fresh_lane())), buf, fresh_lane);
       }
-      for (; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
+      if (i < s) {
+        rescale<Pair>(res, -kOperandScale);
+        for (; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
+      }
       lane = fresh_lane();
     }
 

@@ -1,11 +1,13 @@
-"""17 <= n <= 32: products as sums of bf16 parts, and the two places where the kernel leaves them
-for the FP32 instructions: entries below 2^-100 (a part would be subnormal, which bf16 MFMAs read
-as zero) and squarings from the fifth on whose operands reach 2^60 (a low part's product could
-overflow to the opposite infinity).
+"""17 <= n <= 32: products as sums of bf16 parts, where bf16 MFMAs read subnormal operands as zero:
+the operands are scaled so that no part is subnormal, down to the smallest FP32 values.  Squarings
+from the fifth on whose scaled operands reach 2^60 (a low part's product could overflow to the
+opposite infinity) are left to the FP32 instructions.
 
 Tolerance: FP32 sums of at most 2n = 64 terms over 7 + s products, each squaring doubling the
 relative error: 2^s * 32 * 2^-24 of the Frobenius norm, 2^s * 1.9e-6; measured at most a tenth.
 """
+
+import math
 
 import pytest
 import torch
@@ -31,20 +33,22 @@ def _exact(a, g):
     return torch.linalg.matrix_exp(a), torch.linalg.matrix_exp(block)[:, :a.shape[-1], a.shape[-1]:] * size
 
 
+def _squarings(a, g=None):
+    return torch.ops.flash_hypercons._expm_params(a, g)[0][:, 1].cpu().double()
+
+
 def _run(a, g):
     x = a.to(DEV).requires_grad_()
     y = fh.matrix_exp(x)
     (dx,) = torch.autograd.grad(y, x, g.to(DEV))
-    s = (torch.ops.flash_hypercons._expm_params(x.detach())[1].cpu(),
-         torch.ops.flash_hypercons._expm_params(x.detach().mT, g.to(DEV))[1].cpu())
-    return (y.detach().cpu(), dx.cpu()), s
+    return (y.detach().cpu(), dx.cpu()), (_squarings(x.detach()), _squarings(x.detach().mT, g.to(DEV)))
 
 
-def _check(a, g, rows=slice(None)):
+def _check(a, g, slack=0.0, factor=1.0):
     for out, s, want in zip(*_run(a, g), _exact(a, g)):
-        err = (out.double() - want).flatten(1).norm(dim=1) / want.flatten(1).norm(dim=1)
-        bound = 2.0 ** s.double() * 32 * 2.0**-24
-        assert bool((err <= bound)[rows].all()), (err / bound)[rows].max()
+        err = ((out.double() - want).flatten(1).norm(dim=1) - slack) / want.flatten(1).norm(dim=1)
+        bound = 2.0**s * 32 * 2.0**-24 * factor
+        assert bool((err <= bound).all()), (err / bound).max()
 
 
 @pytest.mark.parametrize("n", (17, 31, 32))
@@ -57,12 +61,8 @@ def test_parts_sum_to_fp32(n, scale):
 @pytest.mark.parametrize("power", (-101, -118, -140))
 def test_tiny_gradients_and_entries_keep_fp32_precision(n, power):
     a, g = _matrices(n, 4, 1.0, n - power)
-    if power > -126:
-        _check(a, g * 2.0**power)
-    else:  # subnormal FP32: one unit of 2^-149 an entry and product
-        got = _run(a, g * 2.0**power)[0][1].double()
-        want = _exact(a, g * 2.0**power)[1]
-        assert bool(((got - want).abs() <= 2.0**-149 * 64 * n + want.abs() * 1e-3).all())
+    # Subnormal FP32 results round to half a unit of 2^-149 an entry.
+    _check(a, g * 2.0**power, slack=n * 2.0**-150)
     # A decoupled pair of tiny entries in an ordinary matrix: exp of the block diag(0.5, 0.25) with
     # an upper right entry t is t (e^0.5 - e^0.25) / 0.25 there.
     t = 2.0 ** max(power, -120)
@@ -71,6 +71,32 @@ def test_tiny_gradients_and_entries_keep_fp32_precision(n, power):
     y = _run(a, g)[0][0][1, 0, 1].item()
     want = t * (torch.tensor(0.5).double().exp() - torch.tensor(0.25).double().exp()).item() / 0.25
     assert abs(y - want) <= 4e-6 * abs(want)
+
+
+@pytest.mark.parametrize("n", (17, 32))
+def test_products_of_small_entries_keep_fp32_precision(n):
+    """Entries that only a product of two small ones reaches: exp(a)_02 = a_01 a_12 / 2 for a alone,
+    and e^t times that where the diagonal is t.  A few roundings of 2^-24, each doubled by a squaring."""
+    for low, high in ((30, 35), (50, 55), (55, 60), (58, 61), (60, 65), (63, 62), (20, 103)):
+        a = torch.zeros(2, n, n)
+        a[:, 0, 1], a[:, 1, 2] = 1.3 * 2.0**-low, 1.7 * 2.0**-high
+        a[1, (0, 1, 2), (0, 1, 2)] = 5.0
+        y, s = fh.matrix_exp(a.to(DEV)).cpu(), _squarings(a.to(DEV))
+        want = a[:, 0, 1].double() * a[:, 1, 2].double() / 2 * torch.tensor([0.0, 5.0]).double().exp()
+        err = (y[:, 0, 2].double() - want).abs() / want
+        assert bool((err <= 2.0**s * 32 * 2.0**-24).all()), (low, high, err)
+
+
+@pytest.mark.parametrize("n", (17, 32))
+@pytest.mark.parametrize("shift", (70, 78, 82, 85))
+def test_small_results_and_gradients_at_strong_decay(n, shift):
+    """exp(-shift I + noise): squarings down to entries of 2^-120, and gradients of 2^-90 to 2^-105
+    at -18 I.  The polynomial's value e^-t, t = shift / 2^s <= 3.01, comes from sums of terms up to
+    e^t, so its relative error is up to e^2t times larger; an eighth of that is allowed and a sixth
+    of the bound measured."""
+    a, g = _matrices(n, 4, 0.02, shift + n)
+    _check(a - shift * torch.eye(n), g, factor=math.exp(2 * shift / 2**5) / 8)
+    _check(a - 18.0 * torch.eye(n), g * 2.0 ** (-shift - 20), slack=n * 2.0**-150, factor=math.exp(2 * 18 / 2**3) / 8)
 
 
 @pytest.mark.parametrize("n", (18, 32))
@@ -82,11 +108,11 @@ def test_many_squarings_in_and_out_of_range(n):
     big = torch.zeros(3, n, n)
     for i, top in enumerate((80.0, 88.0, 200.0)):  # 200: finite operands beyond 2^60, then overflow
         big[i].diagonal().copy_(torch.linspace(-1.0, 1.0, n) * top)
-    y, s = fh.matrix_exp(big.to(DEV)).cpu(), torch.ops.flash_hypercons._expm_params(big.to(DEV))[1].cpu()
+    y, s = fh.matrix_exp(big.to(DEV)).cpu(), _squarings(big.to(DEV))
     diag, want = y.diagonal(dim1=-2, dim2=-1).double(), big.double().diagonal(dim1=-2, dim2=-1).exp()
     fits = want < 3.0e38
-    normal = fits & (want > 2.0**-100)
-    bound = (2.0 ** s.double() * 32 * 2.0**-24)[:, None]
-    assert bool((((diag - want).abs() <= bound * want) | ~normal).all())
-    assert bool((diag[:2] > -1e-30).all()) and not bool(diag[:2].isnan().any())
+    # Decaying entries have the factor of the test above, results below 2^-126 a unit of 2^-149.
+    decay = torch.exp(-2 * big.double().diagonal(dim1=-2, dim2=-1) / 2.0 ** s[:, None]) / 8
+    bound = (2.0**s * 32 * 2.0**-24)[:, None] * decay.clamp_min(1)
+    assert bool((((diag - want).abs() <= bound * want + 2.0**-149) | ~fits).all())
     assert diag[2, -1].item() == float("inf")
