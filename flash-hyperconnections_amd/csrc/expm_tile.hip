@@ -812,7 +812,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTileWaves<P
       }
       if (i < s) {
         rescale<Pair>(res, -kOperandScale);
-        for (; i < s; ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
+        for (; i < (Pair ? s - 1 : s); ++i) res = pmm<P, Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
+        if (Pair) res = pmm<P, Pair, !Pair>(ptranspose<P, Pair>(res, buf, fresh_lane()), res);
       }
       lane = fresh_lane();
     }
