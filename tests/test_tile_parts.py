@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import flash_hypercons as fh
+import oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +117,28 @@ def test_many_squarings_in_and_out_of_range(n):
     bound = (2.0**s * 32 * 2.0**-24)[:, None] * decay.clamp_min(1)
     assert bool((((diag - want).abs() <= bound * want + 2.0**-149) | ~fits).all())
     assert diag[2, -1].item() == float("inf")
+
+
+def _structured(n, batch, scale, seed):
+    """Matrices whose products are single terms or short sums."""
+    gen = torch.Generator().manual_seed(seed)
+    dense, g = torch.randn(batch, n, n, generator=gen) * scale, torch.randn(batch, n, n, generator=gen)
+    blocks = torch.block_diag(*[torch.ones(2, 2)] * n)[:n, :n]
+    return g, {"diagonal": dense * torch.eye(n), "pairs": dense * blocks,
+               "bidiagonal": dense * (torch.eye(n) + torch.ones(n, n).triu(1).tril(1))}
+
+
+@pytest.mark.parametrize("n", (17, 32))
+@pytest.mark.parametrize("scale", (0.5, 3.0, 10.0))
+def test_short_sums_are_as_close_to_fp64_as_fp32_chains(n, scale):
+    """The mean error over 512 matrices against that of the oracle's FP32 chains: means of 512 differ
+    by about 4% (a matrix's error spreads as widely as its mean), so 1.15 of it leaves out a third more."""
+    g, kinds = _structured(n, 512, scale, n)
+    for kind, a in kinds.items():
+        direction = g * (a != 0)
+        got = fh.matrix_exp(a.to(DEV)).cpu(), torch.ops.flash_hypercons._frechet(a.to(DEV), direction.to(DEV)).cpu()
+        chain = oracle.torch_matrix_exp(a)[0], oracle.torch_frechet(a, direction)[0]
+        for ours, theirs, want in zip(got, chain, _exact(a.mT, direction)):
+            want = want.mT if ours is got[0] else want
+            mean = [((r.double() - want).flatten(1).norm(dim=1) / want.flatten(1).norm(dim=1)).mean() for r in (ours, theirs)]
+            assert mean[0] <= 1.15 * mean[1], (kind, mean)
