@@ -118,12 +118,20 @@ __device__ __forceinline__ U32x4 pack(const Vec<T>& v) {
 // Stream rows with the nontemporal hint (cache-policy bit 1: "nt" on gfx950).
 constexpr int kStreamPolicy = 2;
 
-__device__ __forceinline__ U32x4 load16(__amdgpu_buffer_rsrc_t rs, int32_t voff) {
-  return __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0, kStreamPolicy);
+// A lane's column in `voff`, the row in `soff`, a scalar register: no VALU work a
+// row (forming (row, column) offsets per token cost the backward at n = 8 and 64
+// BF16 columns 8%), and neither overflows for lanes past the row's end either (a
+// token spans less than 2^31 bytes, in n >= 2 rows).
+__device__ __forceinline__ U32x4 load16(__amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t soff) {
+  return __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, kStreamPolicy);
 }
 
-__device__ __forceinline__ void store16(U32x4 w, __amdgpu_buffer_rsrc_t rs, int32_t voff) {
-  __builtin_amdgcn_raw_buffer_store_b128(w, rs, voff, 0, kStreamPolicy);
+// The row in the vector offset as well: a wide store needs a scalar offset of 0
+// (kStoreSOffset).  A resource a row instead measured 9 to 17% faster at 64 to 256
+// BF16 columns, but 2 to 4% slower at 2048 to 8192.
+__device__ __forceinline__ void store16(U32x4 w, __amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t row) {
+  const uint32_t at = static_cast<uint32_t>(voff) + static_cast<uint32_t>(row);
+  __builtin_amdgcn_raw_buffer_store_b128(w, rs, static_cast<int32_t>(at), kStoreSOffset, kStreamPolicy);
 }
 
 // One lane's vector of a row of which `left` elements remain.  Ragged: rows in
@@ -135,29 +143,29 @@ __device__ __forceinline__ void store16(U32x4 w, __amdgpu_buffer_rsrc_t rs, int3
 // 213 -> 57 (host), 4096 x 4 x 4093 FP32 361 -> 117 and 964 -> 299 (4.6 and
 // 4.5 TB/s), 16384 x 3 x 1538 FP16 195 -> 64 and 506 -> 171.
 template <typename T, bool Ragged>
-__device__ __forceinline__ U32x4 load_vec(__amdgpu_buffer_rsrc_t rs, int32_t voff, int left) {
+__device__ __forceinline__ U32x4 load_vec(__amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t soff, int left) {
   constexpr int V = Vec<T>::V;
-  if constexpr (!Ragged) return left > 0 ? load16(rs, voff) : U32x4{0, 0, 0, 0};
+  if constexpr (!Ragged) return left > 0 ? load16(rs, voff, soff) : U32x4{0, 0, 0, 0};
   U32x4 w{0, 0, 0, 0};
   if (left >= V) {
-    w = load16(rs, voff);
+    w = load16(rs, voff, soff);
   } else {
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-      if (d * (V / 4) < left) w[d] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff + 4 * d, 0, kStreamPolicy);
+      if (d * (V / 4) < left) w[d] = __builtin_amdgcn_raw_buffer_load_b32(rs, voff + 4 * d, soff, kStreamPolicy);
   }
   return w;
 }
 
 template <typename T, bool Ragged>
-__device__ __forceinline__ void store_vec(U32x4 w, __amdgpu_buffer_rsrc_t rs, int32_t voff, int left) {
+__device__ __forceinline__ void store_vec(U32x4 w, __amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t row, int left) {
   constexpr int V = Vec<T>::V;
   if (Ragged ? left >= V : left > 0) {
-    store16(w, rs, voff);
+    store16(w, rs, voff, row);
   } else if constexpr (Ragged) {
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-      if (d * (V / 4) < left) __builtin_amdgcn_raw_buffer_store_b32(w[d], rs, voff + 4 * d, 0, kStreamPolicy);
+      if (d * (V / 4) < left) __builtin_amdgcn_raw_buffer_store_b32(w[d], rs, voff + 4 * d, row, kStreamPolicy);
   }
 }
 
@@ -276,7 +284,7 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
       const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
       for (int k = 0; k < N; ++k)
-        raw[u][k] = load_vec<T, Ragged>(xs, (k * xr_step + c) * es, cols - c);
+        raw[u][k] = load_vec<T, Ragged>(xs, c * es, k * xr_step * es, cols - c);
     }
   };
   exp_tokens<T, N>(a, sh, lane, wave, etile);
@@ -301,7 +309,7 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
             for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
             y.f[v] = acc;
           }
-          store_vec<T, Ragged>(pack<T>(y), ys, (i2 * cols + c) * es, cols - c);
+          store_vec<T, Ragged>(pack<T>(y), ys, c * es, i2 * cols * es, cols - c);
         }
       }
     }
@@ -402,8 +410,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
         const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          xr[u][k] = load_vec<T, Ragged>(xs, (k * xr_step + c) * es, cols - c);
-          gr[u][k] = load_vec<T, Ragged>(gs, (k * gr_step + c) * es, cols - c);
+          xr[u][k] = load_vec<T, Ragged>(xs, c * es, k * xr_step * es, cols - c);
+          gr[u][k] = load_vec<T, Ragged>(gs, c * es, k * gr_step * es, cols - c);
         }
       }
 #pragma unroll
@@ -425,7 +433,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
             for (int r = 1; r < N; ++r) d = __builtin_fmaf(e.v[4 * r + k], gv[r].f[v], d);
             dx.f[v] = d;
           }
-          store_vec<T, Ragged>(pack<T>(dx), ds, (k * cols + c) * es, cols - c);
+          store_vec<T, Ragged>(pack<T>(dx), ds, c * es, k * cols * es, cols - c);
         }
 #pragma unroll
         for (int r = 0; r < N; ++r)
@@ -551,12 +559,12 @@ __device__ __forceinline__ U32x2 pack8(const Vec8<T>& v) {
   return w;
 }
 
-__device__ __forceinline__ U32x2 load8(__amdgpu_buffer_rsrc_t rs, int32_t voff) {
-  return __builtin_amdgcn_raw_buffer_load_b64(rs, voff, 0, kStreamPolicy);
+__device__ __forceinline__ U32x2 load8(__amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t soff) {
+  return __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, kStreamPolicy);
 }
 
-__device__ __forceinline__ void store8(U32x2 w, __amdgpu_buffer_rsrc_t rs, int32_t voff) {
-  __builtin_amdgcn_raw_buffer_store_b64(w, rs, voff, 0, kStreamPolicy);
+__device__ __forceinline__ void store8(U32x2 w, __amdgpu_buffer_rsrc_t rs, int32_t voff, int32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b64(w, rs, voff, soff, kStreamPolicy);
 }
 
 // E of the set's tokens into `etile` (64 floats per token, rows of 8), eight
@@ -617,7 +625,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
         const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
         for (int k = 0; k < N; ++k)
-          raw[u][k] = c < cols ? load16(xs, (k * xr_step + c) * es) : U32x4{0, 0, 0, 0};
+          raw[u][k] = c < cols ? load16(xs, c * es, k * xr_step * es) : U32x4{0, 0, 0, 0};
       }
 #pragma unroll
       for (int u = 0; u < kWideChunks; ++u) {
@@ -635,7 +643,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
             for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e[i2][k], xv[k].f[v], acc);
             y.f[v] = acc;
           }
-          if (c < cols) store16(pack<T>(y), ys, (i2 * cols + c) * es);
+          if (c < cols) store16(pack<T>(y), ys, c * es, i2 * cols * es);
         }
       }
     }
@@ -674,8 +682,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
         const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          xr[u][k] = c < cols ? load8(xs, (k * xr_step + c) * es) : U32x2{0, 0};
-          gr[u][k] = c < cols ? load8(gs, (k * gr_step + c) * es) : U32x2{0, 0};
+          xr[u][k] = c < cols ? load8(xs, c * es, k * xr_step * es) : U32x2{0, 0};
+          gr[u][k] = c < cols ? load8(gs, c * es, k * gr_step * es) : U32x2{0, 0};
         }
       }
 #pragma unroll
@@ -699,7 +707,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
             for (int r = 1; r < N; ++r) d = __builtin_fmaf(col[r], gv[r].f[v], d);
             dx.f[v] = d;
           }
-          if (c < cols) store8(pack8<T>(dx), ds, (k * cols + c) * es);
+          if (c < cols) store8(pack8<T>(dx), ds, c * es, k * cols * es);
         }
 #pragma unroll
         for (int r = 0; r < N; ++r)
