@@ -12,7 +12,7 @@
 //   in flight form one contiguous region of HBM (consecutive tokens per
 //   workgroup put every concurrent access T tokens apart, a power-of-two stride
 //   that costs about 15% of the bandwidth).  T follows the batch (launch_sets):
-//   8 or 16 when there are tokens enough to fill the chip that way, down to one
+//   8 to 64 when there are tokens enough to fill the chip that way, down to one
 //   token a workgroup.  One wavefront to 8 tokens, however few there were, left
 //   most of the chip idle below 16384 tokens: 64 x 4 x 4096 BF16 forward 61 ->
 //   6.3 us, 2048 x 4 x 4096 forward 80 -> 27 us and backward 132 -> 47 us,
@@ -21,7 +21,7 @@
 //   turn (column_parts), so that one token already keeps four wavefronts
 //   streaming.  The split depends on C alone, so a token's results do not
 //   depend on the batch.
-// * Lane l of every wavefront computes exp(H) of the set's token l with the
+// * Lane l of a wavefront computes exp(H) of its l-th token with the
 //   per-lane P == 4 code (p4_lane.h, the same arithmetic as the
 //   matrix-exponential kernel, so E is bit-identical to it) and parks it in the
 //   wavefront's own LDS.
@@ -50,7 +50,8 @@ namespace {
 using namespace p4;
 
 constexpr int kWaves = 4;    // wavefronts per workgroup
-constexpr int kTokens = 16;  // tokens per workgroup, at most
+constexpr int kTokens = 16;  // tokens per wavefront, at most; per workgroup where its wavefronts share them
+constexpr int kWideTokens = 8;  // the same at n = 5..8, where a set has no exponential to share
 
 struct HcArgs {
   Operand h;        // [B, n, n]
@@ -220,24 +221,25 @@ __device__ __forceinline__ M4 exp_of_token(const Operand& h, int64_t b, bool val
   return e;
 }
 
-// exp(H) of the set's tokens into the wavefront's `etile` (16 floats per
-// token): lane l computes token l (lanes past the set a zero matrix).  `aux`
-// (optional) receives it in FP32 from the first wavefront.
+// exp(H) of the wavefront's tokens into its `etile` (16 floats per token): lane
+// l computes the l-th of them (lanes past the last a zero matrix).  `aux`
+// (optional) receives it in FP32 from one of the wavefronts that share a token.
 template <typename T, int N>
-__device__ __forceinline__ void exp_tokens(const HcArgs& a, const Share& sh, int lane, int wave, float* etile) {
-  const bool valid = sh.holds(lane);
-  const int64_t b = sh.token(lane);
+__device__ __forceinline__ void exp_tokens(const HcArgs& a, const Share& sh, int lane, float* etile, float* aux) {
+  const int slot = sh.first + (lane << sh.shift);
+  const bool valid = sh.holds(slot);
+  const int64_t b = sh.token(slot);
   const M4 e = exp_of_token<T, N>(a.h, b, valid);
   if (valid) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       *reinterpret_cast<float4*>(etile + 16 * lane + 4 * q) =
           make_float4(e.v[4 * q], e.v[4 * q + 1], e.v[4 * q + 2], e.v[4 * q + 3]);
-    if (a.aux && wave == 0) {
+    if (aux && sh.part == 0) {
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int j = 0; j < N; ++j) a.aux[b * N * N + i * N + j] = e.v[4 * i + j];
+        for (int j = 0; j < N; ++j) aux[b * N * N + i * N + j] = e.v[4 * i + j];
     }
   }
   lds_order();
@@ -287,9 +289,9 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
         raw[u][k] = load_vec<T, Ragged>(xs, c * es, k * xr_step * es, cols - c);
     }
   };
-  exp_tokens<T, N>(a, sh, lane, wave, etile);
+  exp_tokens<T, N>(a, sh, lane, etile, a.aux);
   for (int i = sh.first; sh.holds(i); i += sh.abreast) {
-    const M4 e = read_token(etile, i);
+    const M4 e = read_token(etile, i >> sh.shift);
     const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, sh.token(i) * N * a.cols, N * a.cols * es);
     for (int m = 0; sh.column(m, 64 * V) < cols; m += kChunks) {
       load(i, m);
@@ -392,10 +394,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
   const int cols = static_cast<int>(a.cols);
   const int xr_step = static_cast<int>(a.xr);
   const int gr_step = static_cast<int>(a.gr);
-  exp_tokens<T, N>(a, sh, lane, wave, etile);
+  exp_tokens<T, N>(a, sh, lane, etile, nullptr);
   for (int i = sh.first; sh.holds(i); i += sh.abreast) {
     const int64_t b = sh.token(i);
-    const M4 e = read_token(etile, i);
+    const M4 e = read_token(etile, i >> sh.shift);
     const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, b * a.xb, ((N - 1) * a.xr + a.cols) * es);
     const __amdgpu_buffer_rsrc_t gs = rebased<T>(a.gy, b * a.gb, ((N - 1) * a.gr + a.cols) * es);
     const __amdgpu_buffer_rsrc_t ds = rebased<T>(a.out, b * N * a.cols, N * a.cols * es);
@@ -575,8 +577,8 @@ template <int N, bool Transposed>
 __device__ __forceinline__ void load_set_e(const WideArgs& a, const Share& sh, int lane, float* etile) {
   const bool shared = sh.parts > 1;
   const int p = threadIdx.x & 7;
-  for (int t = (shared ? threadIdx.x : lane) >> 3; t < sh.slots; t += shared ? 8 * kWaves : 8) {
-    const int j = shared ? t : sh.first + t * sh.abreast;
+  const int step = shared ? 8 * kWaves : 8 * sh.abreast;
+  for (int j = shared ? threadIdx.x >> 3 : sh.first + (lane >> 3) * sh.abreast; j < sh.slots; j += step) {
     if (p < N && sh.holds(j)) {
       const float* src = a.e + sh.token(j) * (N * N);
 #pragma unroll
@@ -601,7 +603,7 @@ __device__ __forceinline__ void read_row8(const float* tile, int token, int r, f
 // Forward: row i of Y = sum_k E[i][k] X[k] (fmaf chain k = 0..n-1 from +0).
 template <typename T, int N>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_wide_fwd_kernel(WideArgs a) {
-  __shared__ __attribute__((aligned(16))) float etile[kTokens * 64];
+  __shared__ __attribute__((aligned(16))) float etile[kWaves * kWideTokens * 64];
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
   constexpr int V = Vec<T>::V;
   const int lane = threadIdx.x & 63;
@@ -655,8 +657,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
 // wave_sum, then the wavefronts' parts in order), written to a.de.
 template <typename T, int N>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void hc_wide_bwd_kernel(WideArgs a) {
-  __shared__ __attribute__((aligned(16))) float etile[kTokens * 64];
-  __shared__ float gtile[kWaves][kTokens * 64];  // dE by column part
+  // E of the set and, where wavefronts share tokens (a set has kWideTokens then), dE
+  // by column part.
+  __shared__ __attribute__((aligned(16))) float etile[(1 + kWaves) * kWideTokens * 64];
+  float(*const gtile)[kWideTokens * 64] = reinterpret_cast<float(*)[kWideTokens * 64]>(etile + kWideTokens * 64);
   constexpr int es = static_cast<int>(sizeof(typename T::storage));
   constexpr int V = Vec8<T>::V;
   const int lane = threadIdx.x & 63;
@@ -750,9 +754,20 @@ hipError_t launch_sets(void (*kernel)(Args), Args a, int most, hipStream_t strea
   return hipGetLastError();
 }
 
-// Largest sets, BF16, 40000 x 4 x 1024 and 16384 x 4 x 1024, us: forward
-// 8 / 16 / 32 tokens 112 / 116 / 122 and 49.5 / 49.8 / 49.7; backward, which
-// has a Frechet polynomial a set as well, 195 / 178 / 183 and 87 / 81 / 79.
+// Tokens of a wavefront that shares none, at most: as many as have 4 KiB of one row
+// together (what a pass takes of a row that wide), but 2 and no more than `most`.
+// An exponential pass serves a wavefront's tokens however few they are, so sets
+// have to grow as rows shrink: forward 262144 x 4 x C BF16, us, 2 / 4 / 8 / 16
+// tokens, C = 64 264 / 213 / 185 / 174, C = 256 301 / 248 / 223 / 222; 131072 x 4
+// x 512 196 / 180 / 183, 40000 x 4 x 1024 112 / 116 / 122.
+int own_tokens(int64_t row_bytes, int most) {
+  const int64_t each = 4096 / row_bytes;
+  return each < 2 ? 2 : each > most ? most : static_cast<int>(each);
+}
+
+// Where wavefronts share a token, or share the backward's Frechet polynomial a set:
+// 8 / 16 / 32 tokens, 40000 x 4 x 1024 and 16384 x 4 x 1024 BF16 backward 195 / 178 /
+// 183 and 87 / 81 / 79 us.
 template <typename T, int N, bool Backward>
 hipError_t launch_one(HcArgs a, hipStream_t stream) {
   // Whole 16-byte vectors everywhere, or rows in whole dwords at any dword.  The
@@ -766,7 +781,10 @@ hipError_t launch_one(HcArgs a, hipStream_t stream) {
                                : (ragged ? hc_mix_fwd_kernel<T, N, true> : hc_mix_fwd_kernel<T, N, false>);
   // A ragged row shares its columns as the row padded to whole vectors would.
   a.parts = column_parts((a.cols + V - 1) / V * V, 64 * V * kChunksBwd);
-  return launch_sets(kernel, a, Backward ? kTokens : kTokens / 2, stream);
+  const int most = Backward        ? kTokens
+                   : a.parts > 1 ? kTokens / 2
+                                 : kWaves * own_tokens(a.cols * static_cast<int64_t>(sizeof(typename T::storage)), kTokens);
+  return launch_sets(kernel, a, most, stream);
 }
 
 template <typename T>
@@ -781,16 +799,18 @@ hipError_t launch_t(const HcArgs& a, bool backward, hipStream_t stream) {
   }
 }
 
-// n = 5..8, the same at 16384 x 6 x 1024 and 16384 x 8 x 512: forward 8 / 16
-// tokens 68.7 / 70.6 and 47.3 / 46.4 us; backward 103 / 108 and, where a
-// wavefront has a single pass of a token, 83 / 80 us.
+// n = 5..8, where sets cost a load of E: 2 / 4 / 8 / 16 tokens a wavefront at 262144 x
+// 8 x 64 BF16, us, forward 441 / 423 / 407 / 404 and backward 701 / 677 / 656 / 648,
+// but at 100000 x 6 x 128 95 / 92 / 96 / 104 and 181 / 166 / 170 / 188; 8 / 16 tokens
+// a workgroup at 16384 x 6 x 1024 forward 68.7 / 70.6 and backward 103 / 108.
 template <typename T, int N, bool Backward>
 hipError_t launch_wide_one(WideArgs a, hipStream_t stream) {
   const auto kernel = Backward ? hc_wide_bwd_kernel<T, N> : hc_wide_fwd_kernel<T, N>;
   constexpr int pass = 64 * (Backward ? Vec8<T>::V * kWideChunksBwd : Vec<T>::V * kWideChunks);
   // The backward's reduction of 64 sums costs a fifth of a pass: two passes per wavefront at least.
   a.parts = column_parts(a.cols, Backward ? 2 * pass : pass);
-  return launch_sets(kernel, a, Backward && a.cols <= pass ? kTokens : kTokens / 2, stream);
+  const int64_t row_bytes = a.cols * static_cast<int64_t>(sizeof(typename T::storage));
+  return launch_sets(kernel, a, a.parts > 1 ? kWideTokens : kWaves * own_tokens(row_bytes, kWideTokens), stream);
 }
 
 template <typename T, bool Backward>

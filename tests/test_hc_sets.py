@@ -47,3 +47,24 @@ def test_column_shares_and_set_sizes(n, dtype):
             assert bound_violations(y[at], e64 @ x64, e64.abs() @ x64.abs(), n, dtype) == 0, (c, b)
             assert bound_violations(dx[at], e64.mT @ g64, e64.abs().mT @ g64.abs(), n, dtype) == 0, (c, b)
             assert bound_violations(de[at], g64 @ x64.mT, g64.abs() @ x64.abs().mT, dE_terms(c), torch.float32) == 0, (c, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("n", [2, 4, 5, 8])
+def test_largest_sets_of_narrow_rows(n, dtype):
+    """Rows up to 4 KiB are not shared, and a wavefront's tokens grow as rows shrink, to 16 (n <= 4)
+    or 8: whole batches against their pieces, which have smaller sets, bit for bit."""
+    torch.manual_seed(n)
+    for row, b in ((16, 40001), (256, 36863), (512, 33000), (1024, 20000)):
+        c = row // dtype.itemsize
+        h = (torch.randn(b, n, n, device="cuda") * 0.5).to(dtype)
+        x, g = (torch.randn(b, n, c, device="cuda").to(dtype) for _ in range(2))
+        if n <= 4:
+            run = lambda s: (*OPS._hc_mix_aux(h[s], x[s], None)[::2], *OPS._hc_mix_aux(h[s], x[s], g[s]))  # noqa: E731
+        else:
+            e = OPS._matrix_exp(h.float())
+            run = lambda s: (OPS._hc_apply(e[s], x[s]), *OPS._hc_apply_backward(e[s], x[s], g[s]))  # noqa: E731
+        pieces = [run(slice(i, i + 3001)) for i in range(0, b, 3001)]
+        for whole, *parts in zip(run(slice(None)), *pieces):
+            assert same_bits(whole, torch.cat(parts)), (row, b)
