@@ -42,6 +42,8 @@
 // Both directions are bound by HBM traffic (16 FMAs per 2n elements moved
 // forward, 32 per 3n backward); the exponential and Frechet work per token is
 // small beside C >= a few hundred columns.
+#include <type_traits>
+
 #include "p4_lane.h"
 
 namespace fh {
@@ -277,44 +279,53 @@ __global__ __launch_bounds__(64 * kWaves) void hc_mix_fwd_kernel(HcArgs a) {
   // One token's offsets stay below 2^31 (the host checks the spans).
   const int cols = static_cast<int>(a.cols);
   const int xr_step = static_cast<int>(a.xr);
-  // One pass of columns of token i into raw: kChunks chunks from chunk m on.
-  U32x4 raw[kChunks][N];
-  auto load = [&](int i, int m) {
-    const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, sh.token(i) * a.xb, ((N - 1) * a.xr + a.cols) * es);
-#pragma unroll
-    for (int u = 0; u < kChunks; ++u) {
-      const int c = sh.column(m + u, 64 * V) + lane * V;
-#pragma unroll
-      for (int k = 0; k < N; ++k)
-        raw[u][k] = load_vec<T, Ragged>(xs, c * es, k * xr_step * es, cols - c);
-    }
-  };
   exp_tokens<T, N>(a, sh, lane, etile, a.aux);
-  for (int i = sh.first; sh.holds(i); i += sh.abreast) {
-    const M4 e = read_token(etile, i >> sh.shift);
-    const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, sh.token(i) * N * a.cols, N * a.cols * es);
-    for (int m = 0; sh.column(m, 64 * V) < cols; m += kChunks) {
-      load(i, m);
+  // Passes of Chunks chunks.  Ragged rows cost two branches a vector, so chunks past
+  // the row's end are left out: rows of one chunk have passes of one, longer ones
+  // compute and store what is there (a branch between the loads as well costs rows
+  // of 4 KiB 5%).  100000 x 4 x 34, 130 and 258 BF16: 236 -> 88, 238 -> 98 and 239 ->
+  // 106 us (padding the operands instead: 108, 177 and 286).
+  const auto stream = [&](auto chunks) {
+    constexpr int Chunks = decltype(chunks)::value;
+    for (int i = sh.first; sh.holds(i); i += sh.abreast) {
+      const M4 e = read_token(etile, i >> sh.shift);
+      const __amdgpu_buffer_rsrc_t xs = rebased<T>(a.x, sh.token(i) * a.xb, ((N - 1) * a.xr + a.cols) * es);
+      const __amdgpu_buffer_rsrc_t ys = rebased<T>(a.out, sh.token(i) * N * a.cols, N * a.cols * es);
+      for (int m = 0; sh.column(m, 64 * V) < cols; m += Chunks) {
+        U32x4 raw[Chunks][N];
 #pragma unroll
-      for (int u = 0; u < kChunks; ++u) {
-        const int c = sh.column(m + u, 64 * V) + lane * V;
-        Vec<T> xv[N];
+        for (int u = 0; u < Chunks; ++u) {
+          const int c = sh.column(m + u, 64 * V) + lane * V;
 #pragma unroll
-        for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
+          for (int k = 0; k < N; ++k) raw[u][k] = load_vec<T, Ragged>(xs, c * es, k * xr_step * es, cols - c);
+        }
 #pragma unroll
-        for (int i2 = 0; i2 < N; ++i2) {
-          Vec<T> y;
+        for (int u = 0; u < Chunks; ++u) {
+          if (Ragged && sh.column(m + u, 64 * V) >= cols) break;
+          const int c = sh.column(m + u, 64 * V) + lane * V;
+          Vec<T> xv[N];
 #pragma unroll
-          for (int v = 0; v < V; ++v) {
-            float acc = __builtin_fmaf(e.v[4 * i2], xv[0].f[v], 0.f);
+          for (int k = 0; k < N; ++k) xv[k] = unpack<T>(raw[u][k]);
 #pragma unroll
-            for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
-            y.f[v] = acc;
+          for (int i2 = 0; i2 < N; ++i2) {
+            Vec<T> y;
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+              float acc = __builtin_fmaf(e.v[4 * i2], xv[0].f[v], 0.f);
+#pragma unroll
+              for (int k = 1; k < N; ++k) acc = __builtin_fmaf(e.v[4 * i2 + k], xv[k].f[v], acc);
+              y.f[v] = acc;
+            }
+            store_vec<T, Ragged>(pack<T>(y), ys, c * es, i2 * cols * es, cols - c);
           }
-          store_vec<T, Ragged>(pack<T>(y), ys, c * es, i2 * cols * es, cols - c);
         }
       }
     }
+  };
+  if (Ragged && cols <= 64 * V) {
+    stream(std::integral_constant<int, 1>());
+  } else {
+    stream(std::integral_constant<int, kChunks>());
   }
 }
 
