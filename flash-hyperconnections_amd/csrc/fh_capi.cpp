@@ -7,6 +7,7 @@
 #include <string>
 
 #include "fh_kernels.h"
+#include "fh_plan.h"
 #include "fh_rows.h"
 #include "flash_hypercons.h"
 
@@ -203,11 +204,13 @@ Operand hc_operand(const void* h, const int64_t strides[3], int neg, int dtype) 
 }
 
 int64_t compute_units() {
+  static PerDevice units;
   int device = 0;
-  int cus = 0;
   if (hipGetDevice(&device) != hipSuccess) return 1;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 1;
-  return cus > 0 ? cus : 1;
+  return units.get(device, [device] {
+    int cus = 0;
+    return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 0;
+  });
 }
 
 int64_t resident_blocks(const void* kernel, int block) {

@@ -756,7 +756,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
 // balance the last ones, coarser sets pay for fewer exponentials).
 template <typename Args>
 hipError_t launch_sets(void (*kernel)(Args), Args a, int most, hipStream_t stream) {
-  static const int64_t target = 2 * compute_units();
+  const int64_t target = 2 * compute_units();
   const int abreast = kWaves / a.parts;
   const int64_t rounds = (a.batch + target * abreast - 1) / (target * abreast);
   a.tokens = rounds * abreast < most ? static_cast<int>(rounds * abreast) : most;
