@@ -25,4 +25,25 @@ class PerDevice {
   std::atomic<int> values_[kDevices] = {};
 };
 
+// Bytes from the first token's operands of a stream mixing to those of token
+// `first`: h, x and gy by their batch strides (elements of `es` bytes), the
+// contiguous results [B, n, C], [B, n, n] and, in FP32, [B, n, n].
+struct MixBytes {
+  int64_t h, x, gy, rows, square, square_f32;
+};
+inline MixBytes mix_bytes(int64_t first, int64_t es, int64_t n, int64_t cols, int64_t hb, int64_t xb, int64_t gb) {
+  return {first * hb * es, first * xb * es, first * gb * es, first * n * cols * es, first * n * n * es, first * n * n * 4};
+}
+
+// f(first, count) for consecutive slices of at most `most` of `batch` tokens, up to
+// the first that does not return zero.
+template <typename F>
+auto in_slices(int64_t batch, int64_t most, F f) {
+  for (int64_t first = 0;; first += most) {
+    const int64_t left = batch - first;
+    const auto status = f(first, left < most ? left : most);
+    if (static_cast<int>(status) != 0 || left <= most) return status;
+  }
+}
+
 }  // namespace fh

@@ -44,6 +44,7 @@
 // small beside C >= a few hundred columns.
 #include <type_traits>
 
+#include "fh_plan.h"
 #include "p4_lane.h"
 
 namespace fh {
@@ -849,69 +850,57 @@ void* advanced(void* p, int64_t bytes) { return p ? static_cast<char*>(p) + byte
 
 hipError_t launch_hc_apply(const float* e, const void* x, const int64_t* xs, const void* gy, const int64_t* gs,
                            void* out, float* de, int dtype, int64_t batch, int n, int64_t cols, hipStream_t stream) {
-  if (batch > kSlice) {
-    const int64_t es = dtype == F32::code ? 4 : 2;
-    const hipError_t err = launch_hc_apply(e, x, xs, gy, gs, out, de, dtype, kSlice, n, cols, stream);
-    if (err != hipSuccess) return err;
-    return launch_hc_apply(e + kSlice * n * n, advanced(x, kSlice * xs[0] * es), xs,
-                           gy ? advanced(gy, kSlice * gs[0] * es) : nullptr, gs,
-                           advanced(out, kSlice * n * cols * es), de ? de + kSlice * n * n : nullptr, dtype,
-                           batch - kSlice, n, cols, stream);
-  }
-  WideArgs a;
-  a.e = e;
-  a.x = x;
-  a.xb = xs[0];
-  a.xr = xs[1];
-  a.gy = gy;
-  a.gb = gs ? gs[0] : 0;
-  a.gr = gs ? gs[1] : 0;
-  a.out = out;
-  a.de = de;
-  a.batch = batch;
-  a.cols = cols;
-  a.n = n;
-  if (gy != nullptr) {
-    if (dtype == F32::code) return launch_wide_t<F32, true>(a, stream);
-    if (dtype == BF16::code) return launch_wide_t<BF16, true>(a, stream);
-    return launch_wide_t<F16, true>(a, stream);
-  }
-  if (dtype == F32::code) return launch_wide_t<F32, false>(a, stream);
-  if (dtype == BF16::code) return launch_wide_t<BF16, false>(a, stream);
-  return launch_wide_t<F16, false>(a, stream);
+  return in_slices(batch, kSlice, [&](int64_t first, int64_t count) {
+    WideArgs a;
+    a.xb = xs[0];
+    a.xr = xs[1];
+    a.gb = gs ? gs[0] : 0;
+    a.gr = gs ? gs[1] : 0;
+    const MixBytes at = mix_bytes(first, dtype == F32::code ? 4 : 2, n, cols, 0, a.xb, a.gb);
+    a.e = static_cast<const float*>(advanced(e, at.square_f32));
+    a.x = advanced(x, at.x);
+    a.gy = advanced(gy, at.gy);
+    a.out = advanced(out, at.rows);
+    a.de = static_cast<float*>(advanced(de, at.square_f32));
+    a.batch = count;
+    a.cols = cols;
+    a.n = n;
+    if (gy != nullptr) {
+      if (dtype == F32::code) return launch_wide_t<F32, true>(a, stream);
+      if (dtype == BF16::code) return launch_wide_t<BF16, true>(a, stream);
+      return launch_wide_t<F16, true>(a, stream);
+    }
+    if (dtype == F32::code) return launch_wide_t<F32, false>(a, stream);
+    if (dtype == BF16::code) return launch_wide_t<BF16, false>(a, stream);
+    return launch_wide_t<F16, false>(a, stream);
+  });
 }
 
 hipError_t launch_hc_mix(const Operand& h, const void* x, const int64_t* xs, const void* gy, const int64_t* gs,
                          void* out, void* dh, float* aux, int dtype, int64_t batch, int n, int64_t cols,
                          hipStream_t stream) {
-  if (batch > kSlice) {
-    const int64_t es = dtype == F32::code ? 4 : 2;
-    const hipError_t err = launch_hc_mix(h, x, xs, gy, gs, out, dh, aux, dtype, kSlice, n, cols, stream);
-    if (err != hipSuccess) return err;
-    Operand rest = h;
-    rest.data = advanced(h.data, kSlice * h.sb * es);
-    return launch_hc_mix(rest, advanced(x, kSlice * xs[0] * es), xs, gy ? advanced(gy, kSlice * gs[0] * es) : nullptr,
-                         gs, advanced(out, kSlice * n * cols * es), advanced(dh, kSlice * n * n * es),
-                         aux ? aux + kSlice * n * n : nullptr, dtype, batch - kSlice, n, cols, stream);
-  }
-  HcArgs a;
-  a.h = h;
-  a.x = x;
-  a.xb = xs[0];
-  a.xr = xs[1];
-  a.gy = gy;
-  a.gb = gs ? gs[0] : 0;
-  a.gr = gs ? gs[1] : 0;
-  a.out = out;
-  a.dh = dh;
-  a.aux = aux;
-  a.batch = batch;
-  a.cols = cols;
-  a.n = n;
-  const bool backward = gy != nullptr;
-  if (dtype == F32::code) return launch_t<F32>(a, backward, stream);
-  if (dtype == BF16::code) return launch_t<BF16>(a, backward, stream);
-  return launch_t<F16>(a, backward, stream);
+  return in_slices(batch, kSlice, [&](int64_t first, int64_t count) {
+    HcArgs a;
+    a.h = h;
+    a.xb = xs[0];
+    a.xr = xs[1];
+    a.gb = gs ? gs[0] : 0;
+    a.gr = gs ? gs[1] : 0;
+    const MixBytes at = mix_bytes(first, dtype == F32::code ? 4 : 2, n, cols, h.sb, a.xb, a.gb);
+    a.h.data = advanced(h.data, at.h);
+    a.x = advanced(x, at.x);
+    a.gy = advanced(gy, at.gy);
+    a.out = advanced(out, at.rows);
+    a.dh = advanced(dh, at.square);
+    a.aux = static_cast<float*>(advanced(aux, at.square_f32));
+    a.batch = count;
+    a.cols = cols;
+    a.n = n;
+    const bool backward = gy != nullptr;
+    if (dtype == F32::code) return launch_t<F32>(a, backward, stream);
+    if (dtype == BF16::code) return launch_t<BF16>(a, backward, stream);
+    return launch_t<F16>(a, backward, stream);
+  });
 }
 
 }  // namespace fh
