@@ -195,20 +195,24 @@ __device__ __forceinline__ PTm<P, Pair> ptranspose(const PTm<P, Pair>& a, float*
 // An FP32 value is the exact sum of three bf16 values, v = h + m + l with
 // |m| <= 2^-8 |v| and |l| <= 2^-16 |v|, and X.Y is the six products
 //   xh.yh + (xm.yh + xh.ym) + (xl.yh + xm.ym + xh.yl)
-// (the three left out are below 2^-24 |x||y|), summed smallest first in one
-// FP32 accumulator.  Products of bf16 values are exact and an instruction sums 16
-// of them before it rounds, so the result is closer to the exact product than the
-// FP32 instructions' chain: over 512 products of N(0, 1) matrices 3.8e-8 against
-// 1.03e-7 relative error in the 2-norm (cutting values instead of rounding them
-// to their parts gave that advantage away over a whole exponential).
+// (Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype
+// for Higher-Precision Computations", ARITH 2019; the three left out add up to at
+// most 2^-24 |x||y|), summed smallest first in FP32.  Products of bf16 values are
+// exact and an instruction sums 16 of them before it rounds, so results of long
+// sums are closer to the exact product than the FP32 instructions' chain: over 512
+// products of N(0, 1) matrices 3.8e-8 against 1.03e-7 relative error in the 2-norm
+// (cutting values instead of rounding them to their parts gave that advantage away
+// over a whole exponential); short sums are as close (split_pmm).
 //
 // Six bf16 instructions take 3/8 of the FP32 ones' cycles; splitting a matrix
-// costs 16 conversions, shifts or masks and subtractions a lane and part.
-// 32768 32 x 32 FP16 matrices, norms over 1.8 decades, forward + Frechet:
-// 577 -> 409 us (288 + 1061 -> 190 + 622 thousand cycles; the chip runs this
-// kernel at 1.9 GHz, the FP32 one at 2.3).  P = 16 keeps the FP32 instructions:
-// its products are shorter against the splits (341 -> 329 thousand cycles, at the
-// lower clock 150 -> 170 us over 65536 matrices).
+// costs 16 conversions, shifts or masks and subtractions a lane and part, so that
+// a matrix takes 1412 and 3224 VALU instructions (forward, Frechet) for 593 and 1104
+// before, and the matrix pipe is busy 38 and 48% of the time for 75 and 82%.
+// 32768 32 x 32 FP16 matrices N(0, 1) / sqrt(32), forward + Frechet: 143 + 478 ->
+// 111 + 333 us (328 + 1113 -> 223 + 672 thousand cycles, the chip at 2.0 GHz for
+// 2.3); a step over norms of 1.8 decades 581 -> 420 us.  P = 16 keeps the FP32
+// instructions: its products are shorter against the splits (a trial: 150 -> 170 us
+// over 65536 matrices).
 //
 // The k index is permuted as for the FP32 instructions: the B operand of Y
 // comes from the lane's own D-layout values, eight to a 32x32x16 instruction.

@@ -199,7 +199,7 @@ def test_layouts_give_the_same_bits(xl, c, dtype):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=str)
 def test_tokens_do_not_depend_on_the_batch(dtype):
-    # 40,000 tokens: more token sets than the grid holds, so the grid-stride loop is used.
+    # 40,000 tokens: sets of the largest size for a row this short.
     h, x = _inputs(40000, 5, 16, dtype)
     g = torch.randn_like(x, dtype=torch.float32).to(dtype)
     e = _exp(h)
