@@ -210,7 +210,7 @@ __device__ __forceinline__ PTm<P, Pair> ptranspose(const PTm<P, Pair>& a, float*
 // before, and the matrix pipe is busy 38 and 48% of the time for 75 and 82%.
 // 32768 32 x 32 FP16 matrices N(0, 1) / sqrt(32), forward + Frechet: 143 + 478 ->
 // 111 + 333 us (328 + 1113 -> 223 + 672 thousand cycles, the chip at 2.0 GHz for
-// 2.3); a step over norms of 1.8 decades 581 -> 420 us.  P = 16 keeps the FP32
+// 2.3, on another box at 1.8); a step over norms of 1.8 decades 581 -> 420 us.  P = 16 keeps the FP32
 // instructions: its products are shorter against the splits (a trial: 150 -> 170 us
 // over 65536 matrices).
 //
@@ -356,12 +356,15 @@ __device__ __forceinline__ v16f madd(const Left<NX>& x, const Parts<NY>& y, v16f
 // Apart: the leading products h.h and the small ones have an accumulator each.  An
 // instruction cuts the smaller of accumulator and products off near the larger
 // one's last bit: one product onto an accumulator of its sign errs by up to 1 ulp
-// and by -0.17 ulp on average, onto zero by half an ulp at most (measured).  With
-// h.h onto the small products' sum, exp of diagonal FP32 matrices of norms to 10
-// was a third further from FP64 than on the FP32 instructions (mean 7.9e-7 against
-// 6.0e-7), apart it is 6.1e-7; dense matrices are closer either way, 1.1e-6 and
-// 1.2e-6 against 1.6e-6.  It costs 32768 x 32 x 32 Frechet 348 -> 361 us, so results
-// in 16 bits, rounded 2^13 times coarser, go without.
+// and by -0.17 ulp on average, onto zero by half an ulp at most (measured).  Apart,
+// short sums gain that and long ones pay for a third rounding.  So the powers of A
+// and the squarings, whose errors add up or double, are formed apart in FP32, and
+// the polynomial's last two products, to which a sum is added, are not.  Mean error
+// against FP64 relative to the FP32 instructions' chains, 2048 matrices, n = 32,
+// entries N(0, 100) on the diagonal / in 2 x 2 blocks / N(0, 100 / n) everywhere:
+// 1.25 / 1.13 / 0.64 with no product apart, 1.02 / 0.99 / 0.65 so, 1.01 / 0.97 / 0.68
+// with all.  With the operands' scale, 32768 matrices forward + Frechet 135 + 370 ->
+// 141 + 384 us.  Results in 16 bits, rounded 2^13 times coarser, go without.
 template <bool Pair, bool Apart, bool WantD = true, int NX, int NY>
 __device__ __forceinline__ PTm<32, Pair> split_pmm(const PLeft<Pair, NX>& x, const PParts<Pair, NY>& y) {
   v16f d = {}, u = {};
@@ -717,9 +720,9 @@ __device__ __forceinline__ PTm<32, Pair> split_polynomial(const PTm<32, Pair>& a
   const PTm<32, Pair> b4 = combine<3, 2 * kB>(a, a2, a3, a6, id);
   const PTm<32, Pair> b3 = combine<2, 2 * kB>(a, a2, a3, a6, id);
   const PTm<32, Pair> b2 = combine<1, kPolynomialScale>(a, a2, a3, a6, id);
-  const PTm<32, Pair> a9 = padd<32, Pair>(split_pmm<Pair, Apart>(x1, y5), b4);
+  const PTm<32, Pair> a9 = padd<32, Pair>(split_pmm<Pair, false>(x1, y5), b4);
   const PLeft<Pair, 3> x9 = to_left<3, Pair>(padd<32, Pair>(b3, a9), unused, at);
-  return padd<32, Pair>(b2, split_pmm<Pair, Apart>(x9, psplit<3, Pair>(a9)));
+  return padd<32, Pair>(b2, split_pmm<Pair, false>(x9, psplit<3, Pair>(a9)));
 }
 
 template <typename T, int P, bool Pair, int XL, int GL, bool Full>
